@@ -49,8 +49,9 @@ struct gr_gemm_args {
   float alpha;
   const void* r = nullptr;        // residual R (GR_EPI_RES), laid out like C
   long long r_sb = 0, r_sm = 0;   // its batch and row strides
-  int ksplit = 1;                 // fp32 GEMM: blockIdx.z takes K part blockIdx.z of ksplit ...
+  int ksplit = 1;                 // K parts; fp32 GEMM: blockIdx.z takes part blockIdx.z ...
   long long c_sz = 0;             // ... and writes it at C + blockIdx.z * c_sz
+  float* ws = nullptr;            // fp16/bf16 K split: the parts' fp32 sums (gr_gemm_store_part)
 };
 
 template <int EPI>
@@ -148,7 +149,74 @@ __device__ __forceinline__ void gr_gemm_store_tile(const gr_gemm_args& a, const 
   }
 }
 
-template <class T, int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI, int STAGES = 2>
+// The K split's partial sums: part p of tile t (batch-major) is the workgroup's
+// accumulators as they stand in registers, [p][t][i][j][q][thread] of 4 floats
+// (registers 4q..4q+3 of block (i, j)), so that every store and every load of
+// the merge is a whole contiguous KiB per wave. Layout private to this file.
+template <int TM, int TN, int NT>
+__device__ __forceinline__ void gr_gemm_store_part(const gr_gemm_args& a, const gr_f32x16 (&acc)[TN][TM],
+                                                   long long part, long long ntile, long long t) {
+  gr_f32x4* w = reinterpret_cast<gr_f32x4*>(a.ws) + (part * ntile + t) * (TN * TM * 4 * NT) + threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        w[((i * TM + j) * 4 + q) * NT] =
+            (gr_f32x4){acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+}
+
+// Merge of a K split's parts: C = act(alpha * sum of the parts), summed in
+// part order. A thread takes 8 consecutive columns of one row: register quads
+// q of lanes l32 and l32 + 32 of one block (i, j).
+template <class T, int BM, int BN, int WGM, int WGN, int EPI>
+__global__ __launch_bounds__(256) void gr_gemm_merge_kernel(gr_gemm_args a, long long ntile, int tiles_n,
+                                                            int tiles_per_batch) {
+  typedef gr_gemm_cfg<BM, BN, 32, WGM, WGN> G;
+  constexpr int NT = G::NT, TM = G::TM, TN = G::TN, UNITS = TN * TM * 4 * (NT / 2);
+  const long long idx = (long long)blockIdx.x * 256 + threadIdx.x;
+  const long long t = idx / UNITS;
+  if (t >= ntile) return;
+  int u = (int)(idx - t * UNITS);
+  const int l32 = u & 31;
+  u >>= 5;
+  const int wave = u % (NT / 64);
+  u /= NT / 64;
+  const int q = u & 3, j = (u >> 2) % TM, i = (u >> 2) / TM;
+  const long long z = t / tiles_per_batch;
+  const int in = (int)(t - z * tiles_per_batch), tm = in / tiles_n, tn = in % tiles_n;
+  const int row = tm * BM + (wave / WGN) * G::WM + j * 32 + l32;
+  const int col = tn * BN + (wave % WGN) * G::WN + i * 32 + 8 * q;
+  if (row >= a.M || col >= a.N) return;
+  const gr_f32x4* w = reinterpret_cast<const gr_f32x4*>(a.ws) + t * (TN * TM * 4 * NT) +
+                      ((i * TM + j) * 4 + q) * NT + wave * 64 + l32;
+  const long long step = ntile * (TN * TM * 4 * NT);
+  gr_f32x4 lo = w[0], hi = w[32];
+#pragma unroll 4
+  for (int p = 1; p < a.ksplit; ++p) {
+    lo += w[p * step];
+    hi += w[p * step + 32];
+  }
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    v[e] = gr_epilogue<EPI>(a.alpha * lo[e]);
+    v[4 + e] = gr_epilogue<EPI>(a.alpha * hi[e]);
+  }
+  gr_u32x4 out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out[e] = gr_pack2f<T>(v[2 * e], v[2 * e + 1]);
+  gr_st16(static_cast<T*>(a.c) + z * a.c_sb + (long long)row * a.c_sm + col, out);
+}
+
+// SPLIT: the grid is a.ksplit K parts of all tiles; a tile's fp32 sums over its
+// part go to a.ws, for gr_gemm_merge_kernel. Every part holds at least one
+// k tile.
+// KTAIL (BK 64): K may also be an odd multiple of 32 (at least 96); the last k
+// tile then starts at K - BK and only its second half is multiplied.
+template <class T, int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI, int STAGES = 2,
+          bool SPLIT = false, bool KTAIL = false>
 __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
   typedef gr_mfma<T> MF;
   typedef typename MF::vec8 vec8;
@@ -163,7 +231,12 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
   // tile walk: grouped rows, XCD-local groups
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   const int ntile = tiles_m * tiles_n;
-  const int bid = gr_xcd_remap(blockIdx.x, ntile);
+  // SPLIT: the parts' tiles one part after another along blockIdx.x
+  int bid = gr_xcd_remap(blockIdx.x, gridDim.x), part = 0;
+  if constexpr (SPLIT) {
+    part = bid / ntile;
+    bid -= part * ntile;
+  }
   const int per_group = GROUP_M * tiles_n;
   const int grp = bid / per_group;
   const int first_m = grp * GROUP_M;
@@ -177,6 +250,19 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
   const T* B = static_cast<const T*>(a.b) + z * a.b_sb +
                (B_KMAJOR ? (long long)tn * BN * a.b_s : (long long)tn * BN);
   const long long b_step = B_KMAJOR ? (long long)BK : (long long)BK * a.b_s;
+  static_assert(!KTAIL || BK == 64, "the tail skips two of four 16-deep k steps");
+  int nk = KTAIL ? (a.K + BK - 1) / BK : a.K / BK, k0 = 0;
+  int half = KTAIL && a.K % BK ? nk - 1 : -1;      // the half-used last k tile
+  if constexpr (SPLIT) {           // this part's k tiles
+    k0 = (int)((long long)nk * part / a.ksplit);
+    nk = (int)((long long)nk * (part + 1) / a.ksplit) - k0;
+    if constexpr (KTAIL) {
+      half -= half < 0 ? 0 : k0;   // (past nk for every part but the last)
+    } else {
+      A += (long long)k0 * BK;
+      B += k0 * b_step;
+    }
+  }
   // valid rows of this tile of C and valid 16-byte chunks of its rows
   const int rows_ok = a.M - tm * BM < BM ? a.M - tm * BM : BM;
   const int cols_ok = a.N - tn * BN < BN ? a.N - tn * BN : BN;
@@ -203,9 +289,10 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
       am[j] = gr_as<vec8>(gr_ld16(cur + row * (BK * 2) + gr_swz<CPR>(row, 2 * ks + g) * 16));
     }
   };
-  auto mma_tile = [&](const char* cur) {
+  auto mma_tile = [&](const char* cur, bool second_half) {
 #pragma unroll
     for (int ks = 0; ks < BK / 16; ++ks) {
+      if (KTAIL && ks < BK / 32 && second_half) continue;
       vec8 bt[TN], am[TM];
       frags(cur, ks, bt, am);
 #pragma unroll
@@ -221,7 +308,6 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
   // tile (the loads of the later tiles stay in flight; a wave's vector memory
   // operations complete in order). The stage a load overwrites held tile
   // kt - 1, whose last reads finished before the previous barrier.
-  const int nk = a.K / BK;
   gr_lds_loader<T, BM, BK, NT> la;
   // A [K, N] B is copied into LDS as laid out in memory ([BK][BN], swizzled for
   // transposing reads) and its fragments are read back with gr_tr_frag; a
@@ -238,8 +324,14 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
                 "a ring deeper than two stages needs whole 16-byte chunks per thread");
   auto load_tile = [&](int kt) {
     char* dst = lds + (kt % STAGES) * G::STAGE;
-    la.load(A + (long long)kt * BK, dst);
-    lb.load(B + (long long)kt * b_step, dst + G::A_BYTES);
+    if constexpr (KTAIL) {
+      const long long k = gr_imin((k0 + kt) * BK, a.K - BK);
+      la.load(A + k, dst);
+      lb.load(B + (B_KMAJOR ? k : k * a.b_s), dst + G::A_BYTES);
+    } else {
+      la.load(A + (long long)kt * BK, dst);
+      lb.load(B + (long long)kt * b_step, dst + G::A_BYTES);
+    }
   };
   // wait until tile `next` has landed, with `ahead` later tiles in flight
   auto wait_for = [&](int ahead) {
@@ -261,13 +353,18 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
     if (kt + STAGES - 1 < nk) load_tile(kt + STAGES - 1);
-    mma_tile(lds + (kt % STAGES) * G::STAGE);
+    mma_tile(lds + (kt % STAGES) * G::STAGE, kt == half);
     // tiles issued beyond kt + 1
     const int last = kt + STAGES - 1 < nk ? kt + STAGES - 1 : nk - 1;
     wait_for(last - (kt + 1) > 0 ? last - (kt + 1) : 0);
     __syncthreads();
   }
 
+  if constexpr (SPLIT) {
+    gr_gemm_store_part<TM, TN, NT>(a, acc, part, (long long)gridDim.y * ntile,
+                                   z * ntile + (long long)tm * tiles_n + tn);
+    return;
+  }
   // epilogue: the main loop's final barrier has retired every operand read
   gr_gemm_store_tile<T, BM, BN, TM, TN, NT, EPI>(a, acc, lds, wm * G::WM, wn * G::WN, tm, tn, z, rows_ok, cols_ok);
 }
@@ -283,12 +380,13 @@ struct gr_gemm_wpe {
   static constexpr int value = EST > 240 ? 1 : 2;
 };
 
-template <class T, int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI, int STAGES = 2>
+template <class T, int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI, int STAGES = 2,
+          bool SPLIT = false, bool KTAIL = false>
 __global__ __launch_bounds__(WGM * WGN * 64)
 __attribute__((amdgpu_waves_per_eu(gr_gemm_wpe<BM, BN, BK, WGM, WGN, B_KMAJOR>::value)))
 void gr_gemm_kernel(gr_gemm_args a) {
   extern __shared__ __attribute__((aligned(16))) char gr_lds[];
-  gr_gemm_body<T, BM, BN, BK, WGM, WGN, B_KMAJOR, EPI, STAGES>(a, gr_lds);
+  gr_gemm_body<T, BM, BN, BK, WGM, WGN, B_KMAJOR, EPI, STAGES, SPLIT, KTAIL>(a, gr_lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -321,7 +419,8 @@ __device__ __forceinline__ void gr_mfma32_acc(gr_f32x16& acc, V a, V b) {
 template <int BK> struct gr_gemm_w4_stages { static constexpr int value = BK == 64 ? 2 : 4; };
 
 // BNT: the tile's columns, 256 (waves of 128 x 128) or 128 (waves of 128 x 64).
-template <class T, bool B_KMAJOR, int EPI, int BK = 64, int BNT = 256>
+// SPLIT as in gr_gemm_body.
+template <class T, bool B_KMAJOR, int EPI, int BK = 64, int BNT = 256, bool SPLIT = false>
 __device__ __forceinline__ void gr_gemm_w4_body(const gr_gemm_args& a, char* lds) {
   typedef gr_mfma<T> MF;
   typedef typename MF::vec8 vec8;
@@ -341,7 +440,12 @@ __device__ __forceinline__ void gr_gemm_w4_body(const gr_gemm_args& a, char* lds
   // tile walk: grouped rows, XCD-local groups (as gr_gemm_body)
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   const int ntile = tiles_m * tiles_n;
-  const int bid = gr_xcd_remap(blockIdx.x, ntile);
+  // SPLIT: the parts' tiles one part after another along blockIdx.x
+  int bid = gr_xcd_remap(blockIdx.x, gridDim.x), part = 0;
+  if constexpr (SPLIT) {
+    part = bid / ntile;
+    bid -= part * ntile;
+  }
   const int per_group = GROUP_M * tiles_n;
   const int grp = bid / per_group;
   const int first_m = grp * GROUP_M;
@@ -355,6 +459,14 @@ __device__ __forceinline__ void gr_gemm_w4_body(const gr_gemm_args& a, char* lds
   const T* B = static_cast<const T*>(a.b) + z * a.b_sb +
                (B_KMAJOR ? (long long)tn * BN * a.b_s : (long long)tn * BN);
   const long long b_step = B_KMAJOR ? (long long)BK : (long long)BK * a.b_s;
+  int nk = a.K / BK;
+  if constexpr (SPLIT) {           // this part's k tiles
+    const int k0 = (int)((long long)nk * part / a.ksplit);
+    const int k1 = (int)((long long)nk * (part + 1) / a.ksplit);
+    A += (long long)k0 * BK;
+    B += k0 * b_step;
+    nk = k1 - k0;
+  }
   const int rows_ok = a.M - tm * BM < BM ? a.M - tm * BM : BM;
   const int cols_ok = a.N - tn * BN < BN ? a.N - tn * BN : BN;
 
@@ -382,7 +494,6 @@ __device__ __forceinline__ void gr_gemm_w4_body(const gr_gemm_args& a, char* lds
   // stale)
   acc_guard();
 
-  const int nk = a.K / BK;
   typedef gr_lds_loader<T, BM, BK, NT> LA;
   typedef typename gr_cond<B_KMAJOR, gr_lds_loader<T, BN, BK, NT>, gr_lds_loader<T, BK, BN, NT, true>>::type LB;
   LA la;
@@ -487,6 +598,11 @@ __device__ __forceinline__ void gr_gemm_w4_body(const gr_gemm_args& a, char* lds
   // does not count wait states after inline assembly), then every wave past
   // its operand reads before the output tile overwrites the stages
   acc_guard();
+  if constexpr (SPLIT) {
+    gr_gemm_store_part<TM, TN, NT>(a, acc, part, (long long)gridDim.y * ntile,
+                                   z * ntile + (long long)tm * tiles_n + tn);
+    return;
+  }
   __syncthreads();
   gr_gemm_store_tile<T, BM, BN, TM, TN, NT, EPI>(a, acc, lds, wm * G::WM, wn * G::WN, tm, tn, z, rows_ok, cols_ok);
 }
@@ -498,9 +614,9 @@ struct gr_gemm_w4_lds {
   static constexpr int value = G::LDS;
 };
 
-template <class T, bool B_KMAJOR, int EPI, int BK = 64, int BNT = 256>
+template <class T, bool B_KMAJOR, int EPI, int BK = 64, int BNT = 256, bool SPLIT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
 void gr_gemm_w4_kernel(gr_gemm_args a) {
   extern __shared__ __attribute__((aligned(16))) char gr_lds[];
-  gr_gemm_w4_body<T, B_KMAJOR, EPI, BK, BNT>(a, gr_lds);
+  gr_gemm_w4_body<T, B_KMAJOR, EPI, BK, BNT, SPLIT>(a, gr_lds);
 }

@@ -6,6 +6,7 @@
 
 #include "gr_gemm.h"
 #include "gr_gemm_f32.h"
+#include "gr_gemm_plan.h"
 #include "gr_host.h"
 #include "grammar_rt.h"
 
@@ -78,6 +79,80 @@ int launch_gemm_w4(const gr_gemm_args& a, int batch, hipStream_t st) {
   return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_gemm launch");
 }
 
+// A 256 x 128 tile of the one-wave body on its own (picked plans only).
+template <class T, bool KM, int EPI, int BK>
+int launch_gemm_w4h(const gr_gemm_args& a, int batch, hipStream_t st) {
+  const long long nblk = (long long)((a.M + 255) / 256) * ((a.N + 127) / 128);
+  if (nblk > 0x7fffffffLL || batch > 65535)
+    return gr::fail(GR_E_ARG, "gr_gemm: grid (%lld tiles, batch %d) out of range", nblk, batch);
+  hipLaunchKernelGGL((gr_gemm_w4_kernel<T, KM, EPI, BK, 128>), dim3((unsigned)nblk, (unsigned)batch), dim3(256),
+                     (gr_gemm_w4_lds<BK, 128>::value), st, a);
+  return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_gemm launch");
+}
+
+// The tile and K split for a shape, when the caller names neither: the one a
+// model of the launch gives the least time.
+//
+// A workgroup takes t0 + tau us per 64-deep k tile, where tau grows from
+// tau_idle to tau_full as the workgroups resident on the chip grow from few
+// to `slots` per CU (they share HBM, L2 and the matrix cores); a launch is
+// its rounds of resident workgroups, bounded below by reading B at the copy
+// rate (less with too few workgroups to cover the latency). A split adds the
+// merge launch (2 us) and the partial sums' round trip at 6 MB/us. The
+// constants are a least-squares fit to 11,600 launches over M 24-4096, N
+// 512-11008, K 512-11008 and up to 16 parts; the pick is within 4 % of the
+// fastest of those (geometric mean over 504 shapes, 42 % at worst), the
+// 256 x 256 tile that every shape took before at 1.94x of it.
+struct TileModel {
+  int bm, bn, slots;
+  double tau_idle, tau_full, t0;
+  bool whole, split;           // compiled without / with a K split
+};
+constexpr TileModel kTiles64[] = {          // 64-deep k tiles
+    {32, 128, 2, 0.20, 0.66, 1.7, true, true},   {64, 128, 2, 0.35, 0.64, 1.6, true, true},
+    {128, 128, 2, 0.54, 1.00, 1.8, true, true},  {256, 128, 1, 0.67, 0.95, 1.3, true, false},
+    {256, 256, 1, 1.10, 1.40, 3.1, true, true},
+};
+constexpr TileModel kTiles32[] = {          // K not a multiple of 64: 32-deep k tiles from 128 rows on
+    {32, 128, 2, 0.20, 0.66, 1.7, true, true},   {64, 128, 2, 0.35, 0.64, 1.6, true, true},
+    {128, 128, 2, 0.96, 1.12, 0.8, true, true},  {256, 128, 1, 0.58, 0.91, 2.1, true, false},
+    {256, 256, 1, 1.05, 1.39, 3.4, true, true},
+};
+
+gr::GemmPlan pick_plan(int batch, int M, int N, int K, size_t ws_max) {
+  gr::GemmPlan best = {256, 256, 1, 0};
+  const int cus = cu_count();
+  if (cus <= 0) return best;
+  double best_t = 1e30;
+  for (const TileModel& m : K % 64 == 0 ? kTiles64 : kTiles32) {
+    // The 32-row tile reads B once per 32 rows: up to 32, or 64 while a short K
+    // leaves the launch bound by its start (M 48, K 1024: 7.1 us against 10.3
+    // on 64 rows; K 4096 x N 11008: 32 against 24). The larger tiles start
+    // at more than half a tile of rows.
+    if (m.bm == 32 ? M > (K <= 1024 ? 64 : 32) : m.bm > 64 && 2 * M <= m.bm) continue;
+    if (m.bm < 128 && K < 64) continue;        // one 64-deep k tile at least
+    const double tiles = (double)batch * ((M + m.bm - 1) / m.bm) * ((N + m.bn - 1) / m.bn);
+    for (int ks = 1; ks <= 16; ks *= 2) {
+      if (ks == 1 ? !m.whole : !m.split || K / ks < 256 || tiles * ks > 2 * cus) continue;
+      const size_t ws = ks == 1 ? 0 : (size_t)ks * (size_t)tiles * m.bm * m.bn * sizeof(float);
+      if (ws > ws_max) continue;
+      const double nk = K / 64.0 / ks, w = tiles * ks, per = (double)cus * m.slots;
+      auto round = [&](double r) { return nk * (m.tau_idle + (m.tau_full - m.tau_idle) * r / per) + m.t0; };
+      const double full = (double)(long long)(w / per), rem = w - full * per;
+      double t = full * round(per) + (rem > 0 ? round(rem) : 0.);
+      const double rate = w * 0.033 < 4.7 ? w * 0.033 : 4.7;           // MB per us
+      const double read = 2e-6 * batch * N * (double)K / rate;
+      if (t < read) t = read;
+      if (ks > 1) t += 2.0 + 2e-6 * (double)ws / 6.0;
+      if (t < best_t) {
+        best_t = t;
+        best = {m.bm, m.bn, ks, ws};
+      }
+    }
+  }
+  return best;
+}
+
 // (block_m, block_n) -> (k tile, wave grid) compiled into the library; the
 // 128x128 and 256x256 tiles take 64-deep k tiles when K allows, else 32.
 template <class T, bool KM, int EPI>
@@ -95,10 +170,19 @@ int dispatch_tile(const gr_gemm_args& a, int batch, int bm, int bn, hipStream_t 
   return gr::fail(GR_E_ARG, "gr_gemm: unsupported tile (block_m=%d, block_n=%d)", bm, bn);
 }
 
+// plan: a picked one (bm, bn are its tile), or null for the caller's tile.
+template <class T, bool KM, int EPI>
+int dispatch_plan(const gr_gemm_args& a, int batch, int bm, int bn, const gr::GemmPlan* plan, hipStream_t st) {
+  if (plan && bm == 256 && bn == 128)
+    return a.K % 64 == 0 ? launch_gemm_w4h<T, KM, EPI, 64>(a, batch, st) : launch_gemm_w4h<T, KM, EPI, 32>(a, batch, st);
+  return dispatch_tile<T, KM, EPI>(a, batch, bm, bn, st);
+}
+
 template <class T>
-int dispatch(const gr_gemm_args& a, int batch, bool km, int epi, int bm, int bn, hipStream_t st) {
+int dispatch(const gr_gemm_args& a, int batch, bool km, int epi, int bm, int bn, const gr::GemmPlan* plan,
+             hipStream_t st) {
 #define GR_CASE(K, E) \
-  if (km == K && epi == E) return dispatch_tile<T, K, E>(a, batch, bm, bn, st);
+  if (km == K && epi == E) return dispatch_plan<T, K, E>(a, batch, bm, bn, plan, st);
   GR_CASE(false, GR_EPI_NONE)
   GR_CASE(false, GR_EPI_RELU)
   GR_CASE(false, GR_EPI_SILU)
@@ -159,9 +243,11 @@ int dispatch_f32(const gr_gemm_args& a, int batch, bool km, int epi, int bm, int
 
 }  // namespace
 
-extern "C" int gr_gemm(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K,
-                       const long long* a_strides, const long long* b_strides, const long long* c_strides,
-                       int b_kmajor, int epilogue, float alpha, int block_m, int block_n, void* stream) {
+namespace {
+
+int gemm(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K, const long long* a_strides,
+         const long long* b_strides, const long long* c_strides, int b_kmajor, int epilogue, float alpha, int block_m,
+         int block_n, void* workspace, size_t workspace_bytes, void* stream) {
   if (!a || !b || !c || !a_strides || !b_strides || !c_strides) return gr::fail(GR_E_ARG, "gr_gemm: null argument");
   if (batch <= 0 || M <= 0 || N <= 0 || K <= 0) return gr::fail(GR_E_ARG, "gr_gemm: sizes must be positive");
   if (dtype != GR_F32 && (N % 8 != 0 || K % 32 != 0))
@@ -189,16 +275,67 @@ extern "C" int gr_gemm(const void* a, const void* b, void* c, int dtype, int bat
   g.K = K;
   g.alpha = alpha;
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == GR_F16) return dispatch<_Float16>(g, batch, b_kmajor != 0, epilogue, block_m, block_n, st);
-  if (dtype == GR_BF16) return dispatch<__bf16>(g, batch, b_kmajor != 0, epilogue, block_m, block_n, st);
+  const bool km = b_kmajor != 0;
+  if ((dtype == GR_F16 || dtype == GR_BF16) && block_m == 0 && block_n == 0 && epilogue >= GR_EPI_NONE &&
+      epilogue <= GR_EPI_SILU) {
+    const size_t have = workspace ? workspace_bytes : 0;
+    const gr::GemmPlan p = pick_plan(batch, M, N, K, have < gr::kGemmWorkspaceMax ? have : gr::kGemmWorkspaceMax);
+    g.ws = static_cast<float*>(workspace);
+    if (p.bm < 128 || p.ks > 1) return gr::launch_gemm_planned(g, dtype, batch, km, epilogue, p, st);
+    if (dtype == GR_F16) return dispatch<_Float16>(g, batch, km, epilogue, p.bm, p.bn, &p, st);
+    return dispatch<__bf16>(g, batch, km, epilogue, p.bm, p.bn, &p, st);
+  }
+  if (dtype == GR_F16) return dispatch<_Float16>(g, batch, km, epilogue, block_m, block_n, nullptr, st);
+  if (dtype == GR_BF16) return dispatch<__bf16>(g, batch, km, epilogue, block_m, block_n, nullptr, st);
   if (dtype == GR_F32) return dispatch_f32(g, batch, b_kmajor != 0, epilogue, block_m, block_n, st);
   return gr::fail(GR_E_ARG, "gr_gemm: dtype %d unsupported (GR_F32, GR_F16 or GR_BF16)", dtype);
 }
 
+int mlp_fwd(const void* x, const void* w1, const void* w2, void* h, void* y, int dtype, int M, int D, int F,
+            int block_m, int block_n, void* workspace, size_t workspace_bytes, void* stream) {
+  const long long xs[2] = {0, D}, w1s[2] = {0, F}, hs[2] = {0, F}, w2s[2] = {0, D}, ys[2] = {0, D};
+  const int rc = gemm(x, w1, h, dtype, 1, M, F, D, xs, w1s, hs, 0, GR_EPI_SILU, 1.0f, block_m, block_n, workspace,
+                      workspace_bytes, stream);
+  if (rc != 0) return rc;
+  return gemm(h, w2, y, dtype, 1, M, D, F, hs, w2s, ys, 0, GR_EPI_NONE, 1.0f, block_m, block_n, workspace,
+              workspace_bytes, stream);
+}
+
+}  // namespace
+
+extern "C" int gr_gemm(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K,
+                       const long long* a_strides, const long long* b_strides, const long long* c_strides,
+                       int b_kmajor, int epilogue, float alpha, int block_m, int block_n, void* stream) {
+  return gemm(a, b, c, dtype, batch, M, N, K, a_strides, b_strides, c_strides, b_kmajor, epilogue, alpha, block_m,
+              block_n, nullptr, 0, stream);
+}
+
+extern "C" size_t gr_gemm_workspace(int dtype, int batch, int M, int N, int K) {
+  if ((dtype != GR_F16 && dtype != GR_BF16) || batch <= 0 || M <= 0 || N <= 0 || K <= 0) return 0;
+  return pick_plan(batch, M, N, K, gr::kGemmWorkspaceMax).ws;
+}
+
+extern "C" int gr_gemm_ws(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K,
+                          const long long* a_strides, const long long* b_strides, const long long* c_strides,
+                          int b_kmajor, int epilogue, float alpha, void* workspace, size_t workspace_bytes,
+                          void* stream) {
+  if ((uintptr_t)workspace & 15) return gr::fail(GR_E_ARG, "gr_gemm_ws: workspace must be 16-byte aligned");
+  return gemm(a, b, c, dtype, batch, M, N, K, a_strides, b_strides, c_strides, b_kmajor, epilogue, alpha, 0, 0,
+              workspace, workspace_bytes, stream);
+}
+
 extern "C" int gr_mlp_fwd(const void* x, const void* w1, const void* w2, void* h, void* y, int dtype, int M,
                           int D, int F, int block_m, int block_n, void* stream) {
-  const long long xs[2] = {0, D}, w1s[2] = {0, F}, hs[2] = {0, F}, w2s[2] = {0, D}, ys[2] = {0, D};
-  int rc = gr_gemm(x, w1, h, dtype, 1, M, F, D, xs, w1s, hs, 0, GR_EPI_SILU, 1.0f, block_m, block_n, stream);
-  if (rc != 0) return rc;
-  return gr_gemm(h, w2, y, dtype, 1, M, D, F, hs, w2s, ys, 0, GR_EPI_NONE, 1.0f, block_m, block_n, stream);
+  return mlp_fwd(x, w1, w2, h, y, dtype, M, D, F, block_m, block_n, nullptr, 0, stream);
+}
+
+extern "C" size_t gr_mlp_fwd_workspace(int dtype, int M, int D, int F) {
+  const size_t up = gr_gemm_workspace(dtype, 1, M, F, D), down = gr_gemm_workspace(dtype, 1, M, D, F);
+  return up > down ? up : down;
+}
+
+extern "C" int gr_mlp_fwd_ws(const void* x, const void* w1, const void* w2, void* h, void* y, int dtype, int M,
+                             int D, int F, void* workspace, size_t workspace_bytes, void* stream) {
+  if ((uintptr_t)workspace & 15) return gr::fail(GR_E_ARG, "gr_mlp_fwd_ws: workspace must be 16-byte aligned");
+  return mlp_fwd(x, w1, w2, h, y, dtype, M, D, F, 0, 0, workspace, workspace_bytes, stream);
 }

@@ -75,9 +75,21 @@ def gemm(a, b, *, epilogue: str = "none", alpha: float = 1.0, b_kmajor: bool = F
     elif tuple(out.shape) != shape or out.dtype != a.dtype:
         raise ValueError("gemm: bad `out` tensor")
     zc, _, _, c_sb, c_sm = _batch_view(out, "out")
-    rc = rt.lib().gr_gemm(
+    L = rt.lib()
+    dtype = rt.dtype_code(a.dtype)
+    need = 0 if block_m or block_n else int(L.gr_gemm_workspace(dtype, za, M, N, K))
+    if need:
+        ws = rt.workspace(need, a.device, stream)
+        rc = L.gr_gemm_ws(
+            ctypes.c_void_p(a.data_ptr()), ctypes.c_void_p(b.data_ptr()), ctypes.c_void_p(out.data_ptr()),
+            dtype, za, M, N, K, rt._ll2(a_sb, a_sm), rt._ll2(b_sb, b_s), rt._ll2(c_sb, c_sm),
+            int(bool(b_kmajor)), EPILOGUES[epilogue], float(alpha), ctypes.c_void_p(ws.data_ptr()), need,
+            rt._stream_ptr(stream))
+        rt.check(rc, "gr_gemm_ws")
+        return out
+    rc = L.gr_gemm(
         ctypes.c_void_p(a.data_ptr()), ctypes.c_void_p(b.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-        rt.dtype_code(a.dtype), za, M, N, K, rt._ll2(a_sb, a_sm), rt._ll2(b_sb, b_s), rt._ll2(c_sb, c_sm),
+        dtype, za, M, N, K, rt._ll2(a_sb, a_sm), rt._ll2(b_sb, b_s), rt._ll2(c_sb, c_sm),
         int(bool(b_kmajor)), EPILOGUES[epilogue], float(alpha), int(block_m), int(block_n),
         rt._stream_ptr(stream))
     rt.check(rc, "gr_gemm")
@@ -105,9 +117,20 @@ def mlp_fwd(x, w1, w2, *, block_m: int = 0, block_n: int = 0, h=None, out=None, 
     for name, t, shp in (("h", h, (M, F)), ("out", out, (M, D))):
         if tuple(t.shape) != shp or not t.is_contiguous() or t.dtype != x.dtype:
             raise ValueError(f"mlp_fwd: bad `{name}` tensor")
-    rc = rt.lib().gr_mlp_fwd(
+    L = rt.lib()
+    dtype = rt.dtype_code(x.dtype)
+    need = 0 if block_m or block_n else int(L.gr_mlp_fwd_workspace(dtype, M, D, F))
+    if need:
+        ws = rt.workspace(need, x.device, stream)
+        rc = L.gr_mlp_fwd_ws(
+            ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(w1.data_ptr()), ctypes.c_void_p(w2.data_ptr()),
+            ctypes.c_void_p(h.data_ptr()), ctypes.c_void_p(out.data_ptr()), dtype,
+            M, D, F, ctypes.c_void_p(ws.data_ptr()), need, rt._stream_ptr(stream))
+        rt.check(rc, "gr_mlp_fwd_ws")
+        return out
+    rc = L.gr_mlp_fwd(
         ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(w1.data_ptr()), ctypes.c_void_p(w2.data_ptr()),
-        ctypes.c_void_p(h.data_ptr()), ctypes.c_void_p(out.data_ptr()), rt.dtype_code(x.dtype),
+        ctypes.c_void_p(h.data_ptr()), ctypes.c_void_p(out.data_ptr()), dtype,
         M, D, F, int(block_m), int(block_n), rt._stream_ptr(stream))
     rt.check(rc, "gr_mlp_fwd")
     return out

@@ -87,7 +87,14 @@ def lib() -> ctypes.CDLL:
         L.gr_selftest_mfma32.argtypes = [vp, vp, vp, vp]
         L.gr_gemm.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, _ll2, _ll2, _ll2, i32, i32,
                               ctypes.c_float, i32, i32, vp]
+        L.gr_gemm_workspace.argtypes = [i32, i32, i32, i32, i32]
+        L.gr_gemm_workspace.restype = sz
+        L.gr_gemm_ws.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, _ll2, _ll2, _ll2, i32, i32,
+                                 ctypes.c_float, vp, sz, vp]
         L.gr_mlp_fwd.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]
+        L.gr_mlp_fwd_workspace.argtypes = [i32, i32, i32, i32]
+        L.gr_mlp_fwd_workspace.restype = sz
+        L.gr_mlp_fwd_ws.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, vp, sz, vp]
         L.gr_attn_fwd_train.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, _ll3, _ll3, _ll3, _ll3,
                                         i32, i32, ctypes.c_float, i32, i32, vp]
         L.gr_attn_bwd_workspace.argtypes = [i32, i32, i32, i32]
@@ -111,6 +118,7 @@ EXPORTED = (
     "gr_plan_set_step", "gr_plan_run", "gr_plan_free", "gr_plan_time", "gr_attn_fwd",
     "gr_selftest_mfma32", "gr_gemm", "gr_mlp_fwd", "gr_attn_decode_workspace", "gr_attn_decode",
     "gr_attn_fwd_train", "gr_attn_bwd_workspace", "gr_attn_bwd", "gr_attn_decode_noalloc",
+    "gr_gemm_workspace", "gr_gemm_ws", "gr_mlp_fwd_workspace", "gr_mlp_fwd_ws",
 )
 
 # Bytes of the per-device scratch array behind gr_attn_decode_noalloc (GR_DECODE_SCRATCH_BYTES).
@@ -202,6 +210,19 @@ def _stream_ptr(stream) -> ctypes.c_void_p:
         import torch
         stream = torch.cuda.current_stream()
     return ctypes.c_void_p(stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream))
+
+
+def workspace(nbytes: int, device, stream=None):
+    """`nbytes` of device memory for a launch on `stream` (the current stream
+    if None), allocated for that stream: once dropped it is only reused by
+    work queued there later."""
+    import torch
+    if stream is None:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    if not hasattr(stream, "cuda_stream"):
+        stream = torch.cuda.ExternalStream(int(stream), device=device)
+    with torch.cuda.stream(stream):
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
 class Plan:

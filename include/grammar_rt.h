@@ -222,7 +222,8 @@ int gr_attn_decode_noalloc(const void* q, const void* k, const void* v, void* o,
  *  Strides are in elements, multiples of 8 (of 4 for GR_F32); batch stride 0 broadcasts.
  *  epilogue: GR_EPI_NONE, GR_EPI_RELU or GR_EPI_SILU, applied to alpha*acc.
  *  (block_m, block_n) in {(128,128), (256,128), (128,256), (256,256)}
- *  (0 = 256). Any M; N a multiple of 8; K a multiple of 32 (the square
+ *  (0 = 256; both 0: for fp16/bf16 the library picks the tile by M, N, K and
+ *  batch, 32 x 128 and 64 x 128 ones included). Any M; N a multiple of 8; K a multiple of 32 (the square
  *  tiles use 64-deep k tiles when K allows). The 256 x 256 tile runs four
  *  waves of 128 x 128 (one per SIMD); the other tiles run eight waves.
  *  With batch 1, a 256 x 256 launch whose last round of workgroups would
@@ -237,12 +238,31 @@ int gr_gemm(const void* a, const void* b, void* c, int dtype, int batch, int M, 
             const long long* a_strides, const long long* b_strides, const long long* c_strides,
             int b_kmajor, int epilogue, float alpha, int block_m, int block_n, void* stream);
 
+/* gr_gemm with block_m = block_n = 0 and device memory to split K over
+ * workgroups where the tiles of C alone would leave CUs idle (few rows, narrow
+ * C): the parts' fp32 sums go through `workspace` (16-byte aligned, at least
+ * gr_gemm_workspace(dtype, batch, M, N, K) bytes; the call overwrites it) and a
+ * second kernel adds them in a fixed order and applies the epilogue. With a
+ * smaller or NULL workspace the call runs without that split.
+ * gr_gemm_workspace is at most 64 MiB, and 0 where no split is picked (GR_F32
+ * among them). No counterpart in the reference. */
+size_t gr_gemm_workspace(int dtype, int batch, int M, int N, int K);
+int gr_gemm_ws(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K,
+               const long long* a_strides, const long long* b_strides, const long long* c_strides,
+               int b_kmajor, int epilogue, float alpha, void* workspace, size_t workspace_bytes, void* stream);
+
 /* MLP block Y = SiLU(X @ W1) @ W2 as two GEMMs, SiLU fused into the first.
  * The grammar's MLP program (run_mlp_search.py:42-127, with silu in place of
  * relu + residual + LayerNorm). X [M][D], W1 [D][F], W2 [F][D], Y [M][D],
  * all row-major and contiguous; h is caller-provided [M][F] workspace. */
 int gr_mlp_fwd(const void* x, const void* w1, const void* w2, void* h, void* y, int dtype, int M,
                int D, int F, int block_m, int block_n, void* stream);
+
+/* gr_mlp_fwd with block_m = block_n = 0 and a workspace for its GEMMs' K
+ * splits, as gr_gemm_ws (both GEMMs use the same memory, one after the other). */
+size_t gr_mlp_fwd_workspace(int dtype, int M, int D, int F);
+int gr_mlp_fwd_ws(const void* x, const void* w1, const void* w2, void* h, void* y, int dtype, int M,
+                  int D, int F, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Self-test of the 32x32x16 MFMA operand/accumulator layout the kernels
  * assume: one wavefront computes D[32][32] = A[32][16] @ B[16][32] (fp16 in,
