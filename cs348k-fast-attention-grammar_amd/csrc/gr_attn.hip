@@ -7,6 +7,7 @@
 #include <thread>
 #include <vector>
 
+#include "gr_attn_groups.h"
 #include "gr_flash_decode.h"
 #include "gr_flash_f32.h"
 #include "gr_flash_w2.h"
@@ -16,16 +17,18 @@
 
 namespace {
 
+// ragged: the last query tile of a head may be part-filled (N a multiple of BN
+// still), as picked plans launch it.
 template <class T, int D, int BN, int NW, int QB, bool CAUSAL, bool KT, bool PIPE = false>
-int launch_flash(const gr_attn_args& a, hipStream_t st) {
+int launch_flash(const gr_attn_args& a, hipStream_t st, bool ragged = false) {
   constexpr int BM = NW * QB * 32;
   constexpr int LDS = gr_flash_lds<D, BN>::BYTES;
   // K/V tiles go straight into LDS when they give every thread the same
   // number of 16-byte chunks (D * BN / 8 per tile), else through registers.
   constexpr bool DIRECT = (D * BN / 8) % (NW * 64) == 0;
-  if (a.N % BM != 0 || a.N % BN != 0)
+  if ((!ragged && a.N % BM != 0) || a.N % BN != 0)
     return gr::fail(GR_E_ARG, "gr_attn_fwd: N=%d must be a multiple of block_m=%d and block_n=%d", a.N, BM, BN);
-  const long long nblk = (long long)a.B * a.H * (a.N / BM);
+  const long long nblk = (long long)a.B * a.H * ((a.N + BM - 1) / BM);
   if (nblk <= 0 || nblk > 0x7fffffffLL) return gr::fail(GR_E_ARG, "gr_attn_fwd: grid size %lld out of range", nblk);
   hipLaunchKernelGGL((gr_flash_fwd_kernel<T, D, BN, NW, QB, CAUSAL, KT, PIPE, true, DIRECT>), dim3((unsigned)nblk),
                      dim3(NW * 64), LDS, st, a);
@@ -54,15 +57,85 @@ int launch_w2h(const gr_attn_args& a, hipStream_t st) {
   return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_fwd launch");
 }
 
+// The shape of a workgroup for a call that names no tile: nw waves of 32
+// queries x kg key groups (gr_attn_groups.h), bn keys per tile.
+//
+// Modelled time of a launch: t0 + max(lat x iterations of the longest
+// workgroup, thr x iterations per CU) + t1 x workgroups per CU, with `thr` the
+// us per iteration that a CU sustains and `lat` the us that one workgroup
+// alone takes. The constants are fitted to 2,300 launches (B H 1-64, N 64-4096,
+// both head dims, fp16 and bf16, causal or not); the pick is within 0.9 % of
+// the fastest shape (geometric mean, 19 % at worst) and takes 0.77x the time
+// of the largest tile that divides N, which ran before. The 256-query tile
+// that divides N is preferred within the model's error (5 %).
+struct AttnShape {
+  int nw, kg, bn;
+  double lat, thr, t0, t1;
+};
+constexpr AttnShape kShapes64[] = {
+    {1, 4, 32, 0.608, 0.432, 3.07, 1.13}, {1, 8, 32, 0.903, 1.027, 3.41, 1.77}, {2, 2, 64, 0.842, 0.621, 2.79, 1.23},
+    {4, 2, 64, 1.175, 1.204, 3.05, 0.81}, {2, 1, 64, 0.735, 0.297, 2.12, 1.35}, {4, 1, 64, 0.772, 0.560, 2.78, 0.62},
+    {8, 1, 64, 1.044, 1.081, 2.76, 0.83},
+};
+constexpr AttnShape kShapes128[] = {
+    {2, 4, 32, 1.297, 1.333, 3.92, 1.37}, {4, 2, 64, 1.989, 1.990, 2.50, 1.81}, {2, 1, 64, 1.287, 0.704, 3.50, 0.67},
+    {4, 1, 64, 1.129, 1.000, 3.05, 0.83}, {8, 1, 64, 1.665, 1.733, 3.73, 0.27},
+};
+// the two-wave bodies at 256 x 64 (gr_flash_w2.h, gr_flash_w2h.h)
+constexpr AttnShape kShapeW2 = {8, 1, 64, 0.653, 0.961, 0.46, 1.19};
+constexpr AttnShape kShapeW2h = {8, 1, 64, 1.080, 1.585, 2.61, 0.71};
+
+// two_wave: a two-wave body takes the 256 x 64 tile of this call.
+AttnShape pick_shape(int D, bool causal, bool two_wave, long long heads, int N) {
+  const int cus = gr::cu_count() > 0 ? gr::cu_count() : 256;
+  AttnShape best = {0, 0, 0, 0, 0, 0, 0};
+  double best_t = 1e30;
+  auto consider = [&](const AttnShape& s) {
+    const int bm = 32 * s.nw;
+    const double w = (double)heads * ((N + bm - 1) / bm), iters = ((N + s.bn - 1) / s.bn + s.kg - 1) / s.kg;
+    double mean = iters, rounds = (double)(long long)((w + cus - 1) / cus);
+    if (causal) {              // longest first, so a part round costs about a quarter
+      mean *= 0.5 + 0.5 * bm / (N > bm ? N : bm);
+      rounds = w <= cus ? 1. : w / cus + 0.25;
+    }
+    const double alone = iters * s.lat, shared = rounds * mean * s.thr;
+    double t = s.t0 + (alone > shared ? alone : shared) + s.t1 * rounds;
+    if (s.nw == 8 && N % 256 == 0) t *= 0.95;
+    if (t < best_t) {
+      best_t = t;
+      best = s;
+    }
+  };
+  if (D == 64)
+    for (const AttnShape& s : kShapes64)
+      if (!(two_wave && s.nw == 8)) consider(s);
+  if (D == 128)
+    for (const AttnShape& s : kShapes128)
+      if (!(two_wave && s.nw == 8)) consider(s);
+  if (two_wave) consider(D == 64 ? kShapeW2 : kShapeW2h);
+  return best;
+}
+
 // Tile configurations compiled into the library: (block_m, block_n) ->
 // (waves, query blocks per wave, key tile). One wave per 32 queries.
-// block_m 0 / block_n 0 pick the largest tiles that divide N (256 x 128 at
-// D = 64, 256 x 64 at D = 128), except 256 x 64 where the two-wave body of
-// gr_flash_w2.h applies (fp16, D = 64, non-causal, N a multiple of 256).
+// block_m = block_n = 0 runs the picked shape (N a multiple of 64); where that
+// is the 256-query tile and it divides N, and where only one of the two is 0,
+// the zero ones are the largest tiles that divide N (256 x 128 at D = 64, 256
+// x 64 at D = 128), except 256 x 64 where the two-wave body of gr_flash_w2.h
+// applies (fp16, D = 64, non-causal, N a multiple of 256).
 template <class T, int D, bool CAUSAL, bool KT>
 int dispatch_tiles(const gr_attn_args& a, int bm, int bn, hipStream_t st) {
-  if (bm == 0) bm = a.N % 256 == 0 ? 256 : a.N % 128 == 0 ? 128 : 64;
   constexpr bool W2 = gr_is_same<T, _Float16>::value && D == 64 && !CAUSAL;
+  if (bm == 0 && bn == 0 && a.N % 64 == 0) {
+    const bool two_wave = a.N % 256 == 0 && (W2 || (D == 128 && KT && a.lse == nullptr));
+    const AttnShape s = pick_shape(D, CAUSAL, two_wave, (long long)a.B * a.H, a.N);
+    if (s.kg > 1)
+      return gr::launch_flash_groups(a, gr_is_same<T, _Float16>::value ? GR_F16 : GR_BF16, D, CAUSAL, KT, s.nw, s.kg, st);
+    if (s.nw == 2) return launch_flash<T, D, 64, 2, 1, CAUSAL, KT>(a, st, true);
+    if (s.nw == 4) return launch_flash<T, D, 64, 4, 1, CAUSAL, KT>(a, st, true);
+    if (a.N % 256 != 0) return launch_flash<T, D, 64, 8, 1, CAUSAL, KT>(a, st, true);
+  }
+  if (bm == 0) bm = a.N % 256 == 0 ? 256 : a.N % 128 == 0 ? 128 : 64;
   if (bn == 0) bn = (W2 && bm == 256 && a.N % 256 == 0) ? 64 : (D == 64 && a.N % 128 == 0) ? 128 : a.N % 64 == 0 ? 64 : 32;
   if constexpr (W2)
     if (bm == 256 && bn == 64 && a.N % 256 == 0 && a.Nq == a.N) return launch_w2<KT>(a, st);

@@ -1,0 +1,16 @@
+// gr_attn_groups.h -- attention forward launches whose workgroups split the
+// keys over groups of waves (gr_flash_fwd_body's KG), compiled in
+// gr_attn_groups.hip.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "gr_flash_fwd.h"
+
+namespace gr {
+
+// nw waves of 32 queries x kg key groups; N a multiple of 64, any remainder of
+// the query tile. (nw, kg) in {(1, 4), (1, 8), (2, 2), (4, 2)} at D = 64,
+// {(2, 4), (4, 2)} at D = 128; dtype GR_F16 (Q pre-scaled) or GR_BF16.
+int launch_flash_groups(const gr_attn_args& a, int dtype, int D, bool causal, bool kt, int nw, int kg, hipStream_t st);
+
+}  // namespace gr

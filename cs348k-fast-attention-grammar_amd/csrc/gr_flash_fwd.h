@@ -352,8 +352,13 @@ __device__ __forceinline__ void gr_flash_qk_from(gr_f32x16 (&s)[BN / 32][QB], co
 // PRESCALE = false keeps fp16 Q as given and scales every score on the VALU
 // instead (as bf16 does): the launch path for fp16 with scale log2(e) > 1,
 // where the pre-scaled Q could overflow.
+//
+// KG > 1 splits the keys over KG groups of NW waves inside the workgroup: group
+// kg takes key tiles kg, kg + KG, ... through its own LDS ring, and group 0
+// merges the groups' O, base and row sum through LDS at the end. Few query
+// tiles then still give every SIMD two waves, at no traffic beyond the CU.
 template <class T, int D, int BN, int NW, int QB, bool CAUSAL, bool KT_LAYOUT, bool PIPE, bool TR = false,
-          bool DIRECT = false, bool SPLIT = false, bool PRESCALE = true>
+          bool DIRECT = false, bool SPLIT = false, bool PRESCALE = true, int KG = 1>
 __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* lds) {
   typedef gr_mfma<T> MF;
   typedef typename MF::vec8 vec8;
@@ -366,8 +371,13 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
   typedef gr_flash_lds<D, BN> L;
   static_assert(BN % 32 == 0 && D % 32 == 0, "tile shape");
   static_assert(!(SPLIT && (CAUSAL || PIPE)), "key split: non-causal, straight schedule");
+  static_assert(KG == 1 || (DIRECT && !PIPE && !SPLIT), "key groups: direct loads, straight schedule");
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);   // key group
+  const int tid = KG == 1 ? (int)threadIdx.x : (int)threadIdx.x - kg * NT;         // thread of the group
+  const int lane = tid & 63, wave = tid >> 6;
+  char* const lds_all = lds;
+  lds += kg * L::BYTES;
   const int g = lane >> 5, l32 = lane & 31;
   const int Nq = a.Nq;
   const int nqt = (Nq + BM - 1) / BM;
@@ -376,7 +386,8 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
     gr_causal_order((int)blockIdx.x, (int)gridDim.x, nqt, bh, qt);
     qt = nqt - 1 - qt;                        // the longest query tiles first
   } else {
-    const int logical = gr_xcd_remap((int)blockIdx.x, (int)gridDim.x);
+    const int logical = KG == 1 ? gr_xcd_remap((int)blockIdx.x, (int)gridDim.x)
+                                : gr_xcd_remap_any((int)blockIdx.x, (int)gridDim.x);
     bh = logical / nqt;
     qt = logical % nqt;
   }
@@ -475,12 +486,25 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
   kl.init(tid, a.k_sn);
   vl.init(tid, a.v_sn);
   // Element offset of key tile t in K (KT layout: a column offset).
-  const long long k_tile = KT_LAYOUT ? (long long)BN : (long long)BN * a.k_sn;
-  const long long v_tile = (long long)BN * a.v_sn;
+  long long k_tile = KT_LAYOUT ? (long long)BN : (long long)BN * a.k_sn;
+  long long v_tile = (long long)BN * a.v_sn;
 
-  const int ntile = CAUSAL ? (q0 + BM + BN - 1) / BN : nkeys / BN;
+  // Tiles of this group, t = 0, 1, ... (key tile t KG + kg), and the
+  // iterations that every group runs (their barriers are the workgroup's).
+  const int ntile_all = CAUSAL ? (gr_imin(q0 + BM, a.N) + BN - 1) / BN : nkeys / BN;
+  const int ntile = KG == 1 ? ntile_all : (ntile_all - kg + KG - 1) / KG;
+  const int niter = KG == 1 ? ntile_all : (ntile_all + KG - 1) / KG;
+  if constexpr (KG > 1) {
+    Kp += kg * k_tile;
+    Vp += kg * v_tile;
+    k_tile *= KG;
+    v_tile *= KG;
+  }
   const int wq_last = qw + QB * 32 - 1;        // this wave's last query
-  auto wave_active = [&](int t) { return !CAUSAL || t * BN <= wq_last; };
+  auto wave_active = [&](int t) {
+    return KG == 1 ? !CAUSAL || t * BN <= wq_last
+                   : qw < Nq && t < ntile && (!CAUSAL || (t * KG + kg) * BN <= wq_last);
+  };
 
   // LDS ring: K_j and V_j live in slot j & 1. With PIPE the scores of tile
   // t+1 are computed during iteration t (on the matrix cores, while tile t's
@@ -489,8 +513,10 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
   // PIPE iteration t reads K_t, V_t and stores K_{t+1}, V_{t+1}.
   constexpr int KAHEAD = PIPE ? 2 : 1;
   if constexpr (DIRECT) {
-    kl.load(Kp, ks0);
-    vl.load(Vp, vt0);
+    if (KG == 1 || ntile > 0) {
+      kl.load(Kp, ks0);
+      vl.load(Vp, vt0);
+    }
     if (PIPE && ntile > 1) kl.load(Kp + k_tile, ks0 + L::KS);
   } else {
     kl.gload(Kp, tid);
@@ -565,7 +591,7 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
       if (pf_k) kl.gload(Kp + (t + KAHEAD) * k_tile, tid);
       if (pf_v) vl.gload(Vp + (t + 1) * v_tile, tid);
     }
-    const int k0 = t * BN;
+    const int k0 = (t * KG + kg) * BN;
     if (wave_active(t)) {
       // this tile's scores (with PIPE they were computed in the previous
       // iteration) and, on the diagonal of a causal block, the mask
@@ -879,14 +905,71 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
     __syncthreads();
   };
 
-  for (int t = 0; t < ntile; t += 2) {
+  for (int t = 0; t < niter; t += 2) {
     if constexpr (PIPE) {
       tile(t, gr_ic<0>{}, sA, sB);
-      if (t + 1 < ntile) tile(t + 1, gr_ic<1>{}, sB, sA);
+      if (t + 1 < niter) tile(t + 1, gr_ic<1>{}, sB, sA);
     } else {
       tile(t, gr_ic<0>{}, sA, sB);
-      if (t + 1 < ntile) tile(t + 1, gr_ic<1>{}, sA, sB);
+      if (t + 1 < niter) tile(t + 1, gr_ic<1>{}, sA, sB);
     }
+  }
+
+  if constexpr (KG > 1) {
+    // The groups' partials, [group - 1][wave][query block]: O as 4 DB quads of
+    // floats per lane, then base and row sum. The loop's last barrier freed
+    // the rings; the second one here frees them again for the O staging.
+    constexpr int PART = 32 * D * 4 + 64 * 8;
+    static_assert((KG - 1) * NW * QB * PART <= KG * L::BYTES, "the partials fit the rings");
+    auto part = [&](int grp, int qb) { return lds_all + (((grp - 1) * NW + wave) * QB + qb) * PART + lane * 16; };
+    if (kg > 0) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        char* w = part(kg, qb);
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr)
+            *reinterpret_cast<gr_f32x4*>(w + (db * 4 + rr) * 1024) =
+                (gr_f32x4){o[db][qb][4 * rr], o[db][qb][4 * rr + 1], o[db][qb][4 * rr + 2], o[db][qb][4 * rr + 3]};
+        *reinterpret_cast<gr_f32x2*>(w + DB * 4096 - lane * 8) = (gr_f32x2){m[qb], l[qb]};
+      }
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        const float unit = CI ? 1.f : c;          // m is in exponents of 2 (CI) or scores
+        gr_f32x2 ml[KG];
+        float mx = m[qb];
+#pragma unroll
+        for (int k = 1; k < KG; ++k) {
+          ml[k] = *reinterpret_cast<const gr_f32x2*>(part(k, qb) + DB * 4096 - lane * 8);
+          mx = fmaxf(mx, ml[k][0]);
+        }
+        const float base = mx == -GR_INF ? 0.f : mx;
+        const float w0 = gr_exp2((m[qb] - base) * unit);
+        l[qb] *= w0;
+#pragma unroll
+        for (int db = 0; db < DB; ++db) o[db][qb] *= w0;
+        m[qb] = mx;
+#pragma unroll
+        for (int k = 1; k < KG; ++k) {
+          const float wk = gr_exp2((ml[k][0] - base) * unit);
+          l[qb] += wk * ml[k][1];
+#pragma unroll
+          for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+              const gr_f32x4 v = *reinterpret_cast<const gr_f32x4*>(part(k, qb) + (db * 4 + rr) * 1024);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o[db][qb][4 * rr + e] += wk * v[e];
+            }
+        }
+      }
+    }
+    __syncthreads();
+    if (kg > 0) return;
   }
 
   if constexpr (SPLIT) {
@@ -973,10 +1056,10 @@ struct gr_flash_wpe {
 // Kernel wrapper used by the prebuilt library; the grammar renderer emits its
 // own wrappers with baked-in shapes around the same body.
 template <class T, int D, int BN, int NW, int QB, bool CAUSAL, bool KT_LAYOUT, bool PIPE, bool TR = false,
-          bool DIRECT = false, bool SPLIT = false, bool PRESCALE = true>
-__global__ __launch_bounds__(NW * 64)
+          bool DIRECT = false, bool SPLIT = false, bool PRESCALE = true, int KG = 1>
+__global__ __launch_bounds__(NW * KG * 64)
 __attribute__((amdgpu_waves_per_eu(gr_flash_wpe<D, BN, NW, QB, KT_LAYOUT, PIPE>::value)))
 void gr_flash_fwd_kernel(gr_attn_args a) {
   extern __shared__ __attribute__((aligned(16))) char gr_lds[];
-  gr_flash_fwd_body<T, D, BN, NW, QB, CAUSAL, KT_LAYOUT, PIPE, TR, DIRECT, SPLIT, PRESCALE>(a, gr_lds);
+  gr_flash_fwd_body<T, D, BN, NW, QB, CAUSAL, KT_LAYOUT, PIPE, TR, DIRECT, SPLIT, PRESCALE, KG>(a, gr_lds);
 }

@@ -232,7 +232,7 @@ __device__ __forceinline__ void gr_gemm_body(const gr_gemm_args& a, char* lds) {
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   const int ntile = tiles_m * tiles_n;
   // SPLIT: the parts' tiles one part after another along blockIdx.x
-  int bid = gr_xcd_remap(blockIdx.x, gridDim.x), part = 0;
+  int bid = gr_xcd_remap_any(blockIdx.x, gridDim.x), part = 0;
   if constexpr (SPLIT) {
     part = bid / ntile;
     bid -= part * ntile;
@@ -441,7 +441,7 @@ __device__ __forceinline__ void gr_gemm_w4_body(const gr_gemm_args& a, char* lds
   const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   const int ntile = tiles_m * tiles_n;
   // SPLIT: the parts' tiles one part after another along blockIdx.x
-  int bid = gr_xcd_remap(blockIdx.x, gridDim.x), part = 0;
+  int bid = SPLIT ? gr_xcd_remap_any(blockIdx.x, gridDim.x) : gr_xcd_remap(blockIdx.x, gridDim.x), part = 0;
   if constexpr (SPLIT) {
     part = bid / ntile;
     bid -= part * ntile;

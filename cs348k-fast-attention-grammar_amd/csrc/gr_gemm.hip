@@ -25,18 +25,6 @@ int launch_gemm(const gr_gemm_args& a, int batch, hipStream_t st) {
   return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_gemm launch");
 }
 
-// Compute units of the current device (0 if unknown), read once per device.
-int cu_count() {
-  static int cache[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (!cache[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess) cache[dev] = n;
-  }
-  return cache[dev];
-}
-
 // The 256 x 256 tile: four waves (one per SIMD) of 128 x 128, the
 // hand-ordered main loop of gr_gemm_w4_body, one workgroup per CU. When the
 // last round of workgroups would leave more than half of the CUs idle (X W1
@@ -51,7 +39,7 @@ int launch_gemm_w4(const gr_gemm_args& a, int batch, hipStream_t st) {
   const long long nblk = (long long)mt * nt;
   if (nblk <= 0 || nblk > 0x7fffffffLL || batch > 65535)
     return gr::fail(GR_E_ARG, "gr_gemm: grid (%lld tiles, batch %d) out of range", nblk, batch);
-  const int cus = cu_count();
+  const int cus = gr::cu_count();
   if (batch == 1 && cus > 0 && nblk > cus) {
     const long long rounds = (nblk + cus - 1) / cus;
     const long long last = nblk - (rounds - 1) * cus;            // workgroups of the last round
@@ -121,7 +109,7 @@ constexpr TileModel kTiles32[] = {          // K not a multiple of 64: 32-deep k
 
 gr::GemmPlan pick_plan(int batch, int M, int N, int K, size_t ws_max) {
   gr::GemmPlan best = {256, 256, 1, 0};
-  const int cus = cu_count();
+  const int cus = gr::cu_count();
   if (cus <= 0) return best;
   double best_t = 1e30;
   for (const TileModel& m : K % 64 == 0 ? kTiles64 : kTiles32) {

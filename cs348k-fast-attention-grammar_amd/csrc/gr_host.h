@@ -12,4 +12,7 @@ namespace gr {
 // Map a HIP status to GR_OK / `code` with a message naming `what`.
 int hip_check(hipError_t e, int code, const char* what);
 
+// Compute units of the current device (0 if unknown), read once per device.
+int cu_count();
+
 }  // namespace gr

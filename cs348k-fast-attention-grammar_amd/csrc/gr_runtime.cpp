@@ -8,6 +8,7 @@
 // (grammar/optimization.py:284-300, bench.py:49-74).
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <string>
@@ -21,6 +22,16 @@ namespace gr {
 int hip_check(hipError_t e, int code, const char* what) {
   if (e == hipSuccess) return GR_OK;
   return fail(code, "%s: %s (%d)", what, hipGetErrorString(e), (int)e);
+}
+
+int cu_count() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+    cache[dev].store(n, std::memory_order_relaxed);
+  return n;
 }
 
 }  // namespace gr

@@ -131,6 +131,10 @@ int gr_plan_time(gr_plan* p, void* stream, int warmup, int iters, int mode, floa
  *  largest of 256 / 128 / 64 dividing N. block_n: keys per tile, 32 / 64 /
  *  128 (128 at D = 64 only), 0 = 128 at D = 64 when it divides N, else 64
  *  or 32, but 64 where the two-wave body below applies at block_m 256.
+ *  Both 0 (N a multiple of 64): the library picks by B * H, N and the CU count
+ *  among those tiles, part-filled last query tiles included, and workgroups of
+ *  32 to 128 queries that split the keys over 2 to 8 groups of waves, for
+ *  grids that would leave CUs idle; N then need not divide the query tile.
  *  fp16 at D = 64, non-causal, 256 x 64 and N a multiple of 256 runs
  *  the kernel with two waves per SIMD and a hand-ordered main loop (160 KiB
  *  of LDS); so does fp16 or bf16 at D = 128 with K transposed, causal or not,
