@@ -51,6 +51,7 @@ struct gr_gemm_args {
   long long r_sb = 0, r_sm = 0;   // its batch and row strides
   int ksplit = 1;                 // K parts; fp32 GEMM: blockIdx.z takes part blockIdx.z ...
   long long c_sz = 0;             // ... and writes it at C + blockIdx.z * c_sz
+  int kgroups = 1;                // fp32 GEMM: 4 = the k-group body on 32 x 32 blocks (gr_gemm_f32.h)
   float* ws = nullptr;            // fp16/bf16 K split: the parts' fp32 sums (gr_gemm_store_part)
 };
 

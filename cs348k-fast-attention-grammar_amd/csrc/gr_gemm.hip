@@ -204,10 +204,41 @@ int launch_gemm_f32(const gr_gemm_args& a, int batch, hipStream_t st) {
   return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_gemm launch");
 }
 
+// 32 x 32 blocks with K over the four waves of a workgroup.
+template <bool KM, int EPI>
+int launch_gemm_f32_groups(const gr_gemm_args& a, int batch, hipStream_t st) {
+  const long long nblk = (long long)(a.M / 32) * (a.N / 32);
+  if (nblk > 0x7fffffffLL || batch > 65535) return gr::fail(GR_E_ARG, "gr_gemm: grid out of range");
+#define GR_F32G(BK)                                                                                              \
+  hipLaunchKernelGGL((gr_gemm_f32_groups_kernel<BK, KM, EPI>), dim3((unsigned)nblk, (unsigned)batch), dim3(256), \
+                     GR_GEMM_F32_GROUPS_LDS, st, a)
+  if (a.K % 16 == 0) GR_F32G(16);
+  else if (a.K % 8 == 0) GR_F32G(8);
+  else return gr::fail(GR_E_ARG, "gr_gemm: fp32 needs K=%d a multiple of 8", a.K);
+#undef GR_F32G
+  return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_gemm launch");
+}
+
+// Whether the k-group body takes a call whose tile is bm x bn: matrix-core
+// cycles per SIMD of the launch's rounds (64 per 32x32x2 MFMA) less than 0.8
+// of the tile's. _gemm_f32_groups in the renderer is the same rule.
+bool f32_groups(const gr_gemm_args& a, int batch, int bm, int bn) {
+  const int cus = gr::cu_count();
+  if (cus <= 0 || a.M % 32 || a.N % 32) return false;
+  const int waves = (bm >= 64 ? 2 : 1) * (bn >= 64 ? 2 : 1);
+  const long long tiles = (long long)batch * ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
+  const long long blocks = (long long)batch * (a.M / 32) * (a.N / 32);
+  const long long chain = (long long)(bm / 32) * (bn / 32) / waves;       // 32 x 32 blocks per wave
+  const int nk = a.K / (a.K % 16 == 0 ? 16 : 8);                          // k tiles, (nk + 3) / 4 per group
+  return 10 * ((blocks + cus - 1) / cus) * ((nk + 3) / 4) < 8 * ((tiles + cus - 1) / cus) * chain * nk;
+}
+
 template <bool KM, int EPI>
 int dispatch_f32_tile(const gr_gemm_args& a, int batch, int bm, int bn, hipStream_t st) {
+  const bool pick = bm == 0 && bn == 0;
   if (bm == 0) bm = a.M % 128 == 0 ? 128 : a.M % 64 == 0 ? 64 : 32;
   if (bn == 0) bn = a.N % 128 == 0 ? 128 : a.N % 64 == 0 ? 64 : 32;
+  if (pick && f32_groups(a, batch, bm, bn)) return launch_gemm_f32_groups<KM, EPI>(a, batch, st);
 #define GR_T(M_, N_) \
   if (bm == M_ && bn == N_) return launch_gemm_f32<M_, N_, KM, EPI>(a, batch, st);
   GR_T(32, 32) GR_T(32, 64) GR_T(32, 128) GR_T(64, 32) GR_T(64, 64) GR_T(64, 128)

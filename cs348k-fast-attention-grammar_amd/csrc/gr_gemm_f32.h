@@ -23,6 +23,17 @@
 //    [BK][BN] B by 8) so the fragment reads of the 16 or 32 lanes that the
 //    LDS serves together fall on distinct banks.
 //  * M, N multiples of the tile, K of BK; row strides multiples of 4 floats.
+//
+// Grids of few tiles (gr_gemm_f32_groups_body). An fp32 32x32x2 MFMA takes 64
+// cycles, so a wave that owns a 32 x 32 block of C and all of K = 1024 is a
+// serial chain of 14 us, and 32 tiles of 64 x 64 leave seven of eight CUs
+// idle. There a workgroup takes one 32 x 32 block instead and its four waves a
+// quarter of K each, merged through LDS. One wave per SIMD and no operand
+// shared between waves, so nothing is staged: fragments come straight from
+// global memory into registers, two k tiles ahead. 256 x 512, K = 1024: 25.1 us
+// on 32 workgroups of 64 x 64, 7.1 us on 128 of 32 x 32; 256 x 1024, K = 512:
+// 14.1 -> 5.2; 512 x 1024, K = 1024: 25.6 -> 17; 1024 x 1024 (256 tiles of 64 x
+// 64) 26 -> 33, so full grids keep their tile.
 #pragma once
 #include "gr_gemm.h"
 
@@ -46,7 +57,7 @@ struct gr_gemm_f32_cfg {
 };
 
 template <int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI>
-__device__ __forceinline__ void gr_gemm_f32_body(const gr_gemm_args& a, char* lds) {
+__device__ __forceinline__ void gr_gemm_f32_tile_body(const gr_gemm_args& a, char* lds) {
   typedef gr_gemm_f32_cfg<BM, BN, BK, WGM, WGN, B_KMAJOR> G;
   constexpr int NT = G::NT, TM = G::TM, TN = G::TN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -181,6 +192,119 @@ __device__ __forceinline__ void gr_gemm_f32_body(const gr_gemm_args& a, char* ld
   }
 }
 
+// LDS bytes of the k-group body: the four waves' 32 x 32 sums.
+constexpr int GR_GEMM_F32_GROUPS_LDS = 4 * 32 * 32 * 4;
+
+// One 32 x 32 block of C per workgroup of four waves; wave kg takes k tiles kg,
+// kg + 4, ... of 16 (8 where KT is). K a multiple of KT; the grid covers
+// (M / 32) (N / 32) blocks; no K split.
+template <int KT, bool B_KMAJOR, int EPI>
+__device__ __forceinline__ void gr_gemm_f32_groups_body(const gr_gemm_args& a, char* lds) {
+  constexpr int BK = KT > 16 ? 16 : KT;
+  constexpr int KB = BK / 8;                   // 8-deep steps per k tile
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+  const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tiles_n = a.N / 32;
+  const int bid = gr_xcd_remap_any((int)blockIdx.x, (int)gridDim.x);
+  const int tm = bid / tiles_n, tn = bid % tiles_n;
+  const long long z = blockIdx.y;
+  // lane (l32, g): row l32 of A's block, column l32 of B's, k = 8 kb + 4 g + t.
+  // A wave-uniform base per k tile and 32-bit lane offsets kept for the whole
+  // loop: the 64-bit products of per-load addresses cost as much issue time
+  // as the MFMAs (105 cycles per MFMA instead of 64).
+  const char* A = reinterpret_cast<const char*>(static_cast<const float*>(a.a) + z * a.a_sb + (long long)tm * 32 * a.a_sm);
+  const char* B = reinterpret_cast<const char*>(
+      static_cast<const float*>(a.b) + z * a.b_sb + (B_KMAJOR ? (long long)tn * 32 * a.b_s : (long long)tn * 32));
+  const long long b_tile = (B_KMAJOR ? 1LL : a.b_s) * BK * 4;        // bytes
+  const unsigned int a_off = (unsigned int)((l32 * a.a_sm + 4 * g) * 4);
+  unsigned int b_off[B_KMAJOR ? 1 : KB * 4];
+  if constexpr (B_KMAJOR) {
+    b_off[0] = (unsigned int)((l32 * a.b_s + 4 * g) * 4);
+  } else {
+#pragma unroll
+    for (int i = 0; i < KB * 4; ++i) b_off[i] = (unsigned int)(((8 * (i / 4) + 4 * g + i % 4) * a.b_s + l32) * 4);
+  }
+  gr_f32x16 acc[2] = {(gr_f32x16)(0.f), (gr_f32x16)(0.f)};   // two chains: consecutive MFMAs are independent
+
+  auto load = [&](int kt, gr_f32x4 (&fa)[KB], gr_f32x4 (&fb)[KB]) {
+    const char* at = A + (long long)kt * (BK * 4);
+    const char* bt = B + kt * b_tile;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      fa[kb] = *reinterpret_cast<const gr_f32x4*>(at + a_off + kb * 32);
+      if constexpr (B_KMAJOR) {
+        fb[kb] = *reinterpret_cast<const gr_f32x4*>(bt + b_off[0] + kb * 32);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) fb[kb][t] = *reinterpret_cast<const float*>(bt + b_off[kb * 4 + t]);
+      }
+    }
+  };
+  auto mma = [&](const gr_f32x4 (&fa)[KB], const gr_f32x4 (&fb)[KB]) {
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        acc[t & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[kb][t], fa[kb][t], acc[t & 1], 0, 0, 0);
+  };
+  // A ring of NB register buffers, NB - 1 tiles in flight. The loop over whole
+  // turns of the ring has no branch (loads past the wave's last tile repeat
+  // it) and its loads stay ahead of the MFMAs they precede, so that the wait
+  // for a buffer is a count of the later loads. 16-deep tiles in three buffers:
+  // 256 x 512 x 1024 in 7.1 us, against 7.9 / 8.1 / 9.1 for 32-deep ones in
+  // two, three, four and 7.2 / 7.5 for 16-deep ones in two, four.
+  constexpr int NB = 3;
+  const int nk = a.K / BK, n = (nk - kg + 3) / 4, last = kg + (n - 1) * 4;   // this wave's tiles: n
+  gr_f32x4 fa[NB][KB], fb[NB][KB];
+  if (n > 0) {
+#pragma unroll
+    for (int i = 0; i < NB - 1; ++i) load(gr_imin(kg + 4 * i, last), fa[i], fb[i]);
+    int kt = kg;
+    for (int turn = n / NB; turn > 0; --turn, kt += 4 * NB) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        load(gr_imin(kt + 4 * (i + NB - 1), last), fa[(i + NB - 1) % NB], fb[(i + NB - 1) % NB]);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(fa[i], fb[i]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NB - 1; ++i)
+      if (i < n % NB) mma(fa[i], fb[i]);
+  }
+
+  // wave q finishes quad q (columns 8q + 4g + 0..3 of the lane's row): the
+  // groups' sums in order
+  gr_f32x4* x = reinterpret_cast<gr_f32x4*>(lds);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    gr_f32x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = acc[0][4 * q + e] + acc[1][4 * q + e];
+    x[(kg * 4 + q) * 64 + lane] = w;
+  }
+  __syncthreads();
+  gr_f32x4 sum = x[kg * 64 + lane];
+#pragma unroll
+  for (int k = 1; k < 4; ++k) sum += x[(k * 4 + kg) * 64 + lane];
+  const long long row = tm * 32 + l32, col = tn * 32 + 8 * kg + 4 * g;
+  gr_f32x4 w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = gr_epilogue<EPI>(a.alpha * sum[e]);
+  if constexpr ((EPI & GR_EPI_RES) != 0)
+    w += *reinterpret_cast<const gr_f32x4*>(static_cast<const float*>(a.r) + z * a.r_sb + row * a.r_sm + col);
+  *reinterpret_cast<gr_f32x4*>(static_cast<float*>(a.c) + z * a.c_sb + row * a.c_sm + col) = w;
+}
+
+// A rendered stage: the program's tile, or (a.kgroups, a constant there) its
+// 32 x 32 blocks on the k-group body, one workgroup of 256 threads each.
+template <int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI>
+__device__ __forceinline__ void gr_gemm_f32_body(const gr_gemm_args& a, char* lds) {
+  if (a.kgroups == 4) gr_gemm_f32_groups_body<BK, B_KMAJOR, EPI>(a, lds);
+  else gr_gemm_f32_tile_body<BM, BN, BK, WGM, WGN, B_KMAJOR, EPI>(a, lds);
+}
+
 // The second launch of a split-K GEMM: C = act(alpha * sum_s P_s) [+ R] over
 // the ksplit partial products P_s (at ws + s * ws_sz, laid out as C with
 // row stride N, batch stride M N). One thread per 4 consecutive columns of
@@ -207,5 +331,11 @@ __device__ __forceinline__ void gr_gemm_f32_reduce_body(const gr_gemm_args& a, c
 template <int BM, int BN, int BK, int WGM, int WGN, bool B_KMAJOR, int EPI>
 __global__ __launch_bounds__(WGM * WGN * 64) void gr_gemm_f32_kernel(gr_gemm_args a) {
   extern __shared__ __attribute__((aligned(16))) char gr_lds[];
-  gr_gemm_f32_body<BM, BN, BK, WGM, WGN, B_KMAJOR, EPI>(a, gr_lds);
+  gr_gemm_f32_tile_body<BM, BN, BK, WGM, WGN, B_KMAJOR, EPI>(a, gr_lds);
+}
+
+template <int BK, bool B_KMAJOR, int EPI>
+__global__ __launch_bounds__(256) void gr_gemm_f32_groups_kernel(gr_gemm_args a) {
+  extern __shared__ __attribute__((aligned(16))) char gr_lds[];
+  gr_gemm_f32_groups_body<BK, B_KMAJOR, EPI>(a, gr_lds);
 }

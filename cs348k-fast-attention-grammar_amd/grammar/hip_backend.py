@@ -526,6 +526,22 @@ def _gemm_f32_lds(bm, bn, bk, kmajor):
     return 2 * 4 * (a + b)
 
 
+GEMM_F32_GROUPS_LDS = 4 * 32 * 32 * 4      # LDS bytes of gr_gemm_f32_groups_body
+
+
+def _gemm_f32_groups(M, N, nk, batch, bm, bn, cus=GEMM_CUS):
+    """Whether an fp32 GEMM stage runs as 32 x 32 blocks with K over the four
+    waves of a workgroup (gr_gemm_f32_groups_body) instead of the program's
+    tile: the library's f32_groups rule, matrix-core cycles per SIMD of the
+    launch's rounds below 0.8 of the tile's (nk k tiles over four groups).
+    64 x 64 tiles with K = 1024: 256 x 512 (32 of them) 25.1 -> 7.1 us, 512 x
+    1024 (128) 25.6 -> 17, 1024 x 1024 (256) 26 -> 33."""
+    waves = (2 if bm >= 64 else 1) * (2 if bn >= 64 else 1)
+    chain = (bm // 32) * (bn // 32) // waves            # 32 x 32 blocks per wave, nk k tiles each
+    tiles = batch * _cdiv(M, bm) * _cdiv(N, bn)
+    return 10 * _cdiv(batch * (M // 32) * (N // 32), cus) * _cdiv(nk, 4) < 8 * _cdiv(tiles, cus) * chain * nk
+
+
 def _gemm_waves(bm, bn):
     wgm, wgn = GEMM_WAVES_M[bm], GEMM_WAVES_N[bn]
     if bm == 256 and bn == 256:
@@ -753,8 +769,13 @@ def _render_gemm(loop, program, f) -> tuple:
         return _render_gemm_f32_split(loop, program, f, args, params, km)
     if f.get("f32"):
         nt = f["WGM"] * f["WGN"] * 64
+        groups = _gemm_f32_groups(f["M"], f["N"], f["K"] // min(f["BK"], 16), f["batch"], f["BM"], f["BN"])
+        how, kg_line = "", ""
+        if groups:
+            nt = 256
+            how, kg_line = ",\n// as 32x32 blocks with K over four waves", "\n  a.kgroups = 4;"
         code = f"""
-// stage {loop.out}: fp32 MFMA GEMM {f['M']}x{f['N']}x{f['K']} (x{f['batch']}), tile {f['BM']}x{f['BN']}x{f['BK']}
+// stage {loop.out}: fp32 MFMA GEMM {f['M']}x{f['N']}x{f['K']} (x{f['batch']}), tile {f['BM']}x{f['BN']}x{f['BK']}{how}
 extern "C" __global__ __launch_bounds__({nt})
 void {kname}({params}) {{
   extern __shared__ __attribute__((aligned(16))) char gr_gemm_smem[];
@@ -764,14 +785,19 @@ void {kname}({params}) {{
   a.b_sb = {f['b_sb']}LL; a.b_s = {f['K'] if f['kmajor'] else f['N']};
   a.c_sb = {f['c_sb']}LL; a.c_sm = {f['N']};
   a.M = {f['M']}; a.N = {f['N']}; a.K = {f['K']};
-  a.alpha = {_flt(f['alpha'])};{res_line}
+  a.alpha = {_flt(f['alpha'])};{res_line}{kg_line}
   gr_gemm_f32_body<{f['BM']}, {f['BN']}, {f['BK']}, {f['WGM']}, {f['WGN']}, {km}, {f['act']}>(a, gr_gemm_smem);
 }}
 """
+        tiles = {"block_m": f["BM"], "block_n": f["BN"], "block_k": f["BK"]}
+        if groups:
+            return code, {"kernel": kname, "grid": [(f["M"] // 32) * (f["N"] // 32), f["batch"], 1],
+                          "block": [nt, 1, 1], "lds": GEMM_F32_GROUPS_LDS, "args": args, "lowering": "gemm",
+                          "tiles": {**tiles, "k_groups": 4}}
         grid = (f["M"] // f["BM"]) * (f["N"] // f["BN"])
         return code, {"kernel": kname, "grid": [grid, f["batch"], 1], "block": [nt, 1, 1],
                       "lds": _gemm_f32_lds(f["BM"], f["BN"], f["BK"], f["kmajor"]), "args": args,
-                      "lowering": "gemm", "tiles": {"block_m": f["BM"], "block_n": f["BN"], "block_k": f["BK"]}}
+                      "lowering": "gemm", "tiles": tiles}
     if f.get("W4"):
         def w4_kernel(name, col0, ncols, bnt, what):
             # columns col0 .. col0 + ncols of C (B, C and R offset by col0)

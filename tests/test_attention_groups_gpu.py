@@ -54,7 +54,7 @@ CASES = [
     (1, 2, 320, 128, "fp16", True, True),     # 2 waves x 4 groups
     (1, 12, 1344, 128, "bf16", False, True),
     (1, 3, 1984, 128, "fp16", False, False),
-    (2, 32, 448, 128, "bf16", True, False),   # 4 waves x 2 groups
+    (2, 32, 384, 128, "bf16", True, False),   # 4 waves x 2 groups
     (1, 12, 1408, 128, "fp16", False, True),
     (2, 12, 1344, 128, "bf16", False, False),  # 64-query tiles, one group
     (2, 32, 1344, 128, "fp16", True, True),   # 256-query causal tiles, ragged
