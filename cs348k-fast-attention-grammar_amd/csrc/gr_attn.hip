@@ -212,58 +212,108 @@ int dispatch_shape(const gr_attn_args& a, int D, bool causal, bool kt, int bm, i
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Merge of the key-split partials: one thread per (head, query, 8 of D).
+// Merge of the key-split partials: one wave per (head, query) row.
 // m_s are the parts' reference maxima (score units), l_s their row sums:
 // O = sum_s w_s O_s / sum_s w_s l_s with w_s = 2^((m_s - max_s m_s) c).
-template <class T, int D>
+// Bound by latency. SPREAD (many parts): a wave per row; lane s holds part s's
+// (m, l), so the weights of 64 parts take one load, and its 64 / (D / 4) groups
+// of lanes take every such part of O, 16 bytes per lane. Else: a group of
+// lanes per row, looping over the few parts. One thread per 8 columns looping
+// over all parts took 7.5 us for 640 rows of 11 parts at D = 64 (here 3.4) and
+// 16 us for 40 rows of 32.
+template <class T, int D, bool SPREAD>
 __global__ __launch_bounds__(256) void gr_attn_combine_kernel(const float* __restrict__ po, const float* __restrict__ pml,
                                                               T* o, long long o_sb, long long o_sh, long long o_sn,
                                                               int B, int H, int Nq, int S, float c) {
-  constexpr int CH = D / 8;
-  const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long rows = (long long)B * H * Nq;
-  if (idx >= rows * CH) return;
-  const int ch = (int)(idx % CH);
-  const long long row = idx / CH;              // (b*H + h) * Nq + q
-  const int q = (int)(row % Nq);
-  const int bh = (int)(row / Nq);
-  const long long stride = rows;               // rows per split
-  float mx = -GR_INF;
-  for (int s = 0; s < S; ++s) mx = fmaxf(mx, pml[(s * stride + row) * 2]);
-  float L = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < S; ++s) {
-    const float* ml = pml + (s * stride + row) * 2;
-    const float w = gr_exp2((ml[0] - mx) * c);
-    L += w * ml[1];
-    const float* src = po + (s * stride + row) * D + ch * 8;
-    const gr_f32x4 v0 = *reinterpret_cast<const gr_f32x4*>(src);
-    const gr_f32x4 v1 = *reinterpret_cast<const gr_f32x4*>(src + 4);
+  constexpr int CH = D / 4, GRP = 64 / CH;
+  const int lane = threadIdx.x & 63, ch = lane % CH, grp = lane / CH;
+  const long long rows = (long long)B * H * Nq;                 // rows per part
+  const long long wave = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long long row = SPREAD ? wave : wave * GRP + grp;       // (b*H + h) * Nq + q
+  if (row >= rows) return;
+  auto part_ml = [&](int s) {
+    return s < S ? *reinterpret_cast<const gr_f32x2*>(pml + (s * rows + row) * 2) : (gr_f32x2){-GR_INF, 0.f};
+  };
+  float mx = -GR_INF, L = 0.f;
+  gr_f32x4 acc = (gr_f32x4)(0.f);
+  if constexpr (SPREAD) {
+    for (int s0 = 0; s0 < S; s0 += 64) mx = fmaxf(mx, part_ml(s0 + lane)[0]);
+    mx = gr_wave_max(mx);
+    const float base = mx == -GR_INF ? 0.f : mx;
+    for (int s0 = 0; s0 < S; s0 += 64) {
+      const gr_f32x2 ml = part_ml(s0 + lane);
+      const float w = gr_exp2((ml[0] - base) * c);
+      L += w * ml[1];
+      const int n = gr_imin(S - s0, 64);
+#pragma unroll 4
+      for (int s = 0; s < n; s += GRP) {
+        const int p = gr_imin(s + grp, n - 1);                  // past the last: its copy, not added
+        const float wp = __shfl(w, p, 64);
+        const gr_f32x4 v = *reinterpret_cast<const gr_f32x4*>(po + ((s0 + p) * rows + row) * D + ch * 4);
+        if (s + grp < n) acc += wp * v;
+      }
+    }
+    L = gr_wave_sum(L);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      acc[e] += w * v0[e];
-      acc[4 + e] += w * v1[e];
+    for (int off = CH; off < 64; off <<= 1)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+    if (grp != 0) return;
+  } else {
+    gr_f32x2 ml[4];            // at most four parts, all loads ahead of the first use
+    gr_f32x4 v[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      ml[s] = part_ml(s);
+      v[s] = *reinterpret_cast<const gr_f32x4*>(po + (gr_imin(s, S - 1) * rows + row) * D + ch * 4);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) mx = fmaxf(mx, ml[s][0]);
+    const float base = mx == -GR_INF ? 0.f : mx;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float w = gr_exp2((ml[s][0] - base) * c);
+      if (s < S) {
+        L += w * ml[s][1];
+        acc += w * v[s];
+      }
     }
   }
   const float inv = 1.0f / L;
-  gr_u32x4 out;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) out[e] = gr_pack2f<T>(acc[2 * e] * inv, acc[2 * e + 1] * inv);
-  const int b = bh / H, h = bh % H;
-  gr_st16(o + b * o_sb + h * o_sh + (long long)q * o_sn + ch * 8, out);
+  const int q = (int)(row % Nq), bh = (int)(row / Nq), b = bh / H, h = bh % H;
+  *reinterpret_cast<gr_u32x2*>(o + b * o_sb + h * o_sh + (long long)q * o_sn + ch * 4) =
+      (gr_u32x2){gr_pack2f<T>(acc[0] * inv, acc[1] * inv), gr_pack2f<T>(acc[2] * inv, acc[3] * inv)};
 }
 
-template <class T, int D, int BN, int NW, bool SPLIT, bool PRESCALE = true>
+template <class T, int D>
+int launch_combine(const gr_attn_args& a, int S, hipStream_t st) {
+  const long long rows = (long long)a.B * a.H * a.Nq;
+  const long long waves = S > 4 ? rows : (rows * (D / 4) + 63) / 64;
+  const dim3 grid((unsigned)((waves + 3) / 4));
+  if (S > 4)
+    hipLaunchKernelGGL((gr_attn_combine_kernel<T, D, true>), grid, dim3(256), 0, st, a.part_o, a.part_ml,
+                       static_cast<T*>(a.o), a.o_sb, a.o_sh, a.o_sn, a.B, a.H, a.Nq, S, a.scale_log2);
+  else
+    hipLaunchKernelGGL((gr_attn_combine_kernel<T, D, false>), grid, dim3(256), 0, st, a.part_o, a.part_ml,
+                       static_cast<T*>(a.o), a.o_sb, a.o_sh, a.o_sn, a.B, a.H, a.Nq, S, a.scale_log2);
+  return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_decode combine launch");
+}
+
+template <class T, int D, int BN, int NW, bool SPLIT, bool PRESCALE = true, int KG = 1>
 void decode_kernel(const gr_attn_args& a, dim3 grid, hipStream_t st) {
-  constexpr int LDS = gr_flash_lds<D, BN>::BYTES;
-  hipLaunchKernelGGL((gr_flash_fwd_kernel<T, D, BN, NW, 1, false, false, false, true, true, SPLIT, PRESCALE>), grid,
-                     dim3(NW * 64), LDS, st, a);
+  constexpr int LDS = KG * gr_flash_lds<D, BN>::BYTES;
+  hipLaunchKernelGGL((gr_flash_fwd_kernel<T, D, BN, NW, 1, false, false, false, true, true, SPLIT, PRESCALE, KG>), grid,
+                     dim3(NW * KG * 64), LDS, st, a);
 }
 
-template <class T, int D, int BN, bool SPLIT>
-void decode_nw(const gr_attn_args& a, int nw, dim3 grid, hipStream_t st) {
-  if (nw == 1) decode_kernel<T, D, BN, 1, SPLIT>(a, grid, st);
-  else if (nw == 2) decode_kernel<T, D, BN, 2, SPLIT>(a, grid, st);
-  else decode_kernel<T, D, BN, 4, SPLIT>(a, grid, st);
+// nw 1 or 2: four key groups of 32-key tiles (a part's keys over 4 or 8 waves);
+// 4: one group of 64-key tiles, or 32 when N is not a multiple of 64.
+template <class T, int D, bool SPLIT>
+void decode_nw(const gr_attn_args& a, int nw, bool bn64, dim3 grid, hipStream_t st) {
+  if (nw == 1) decode_kernel<T, D, 32, 1, SPLIT, true, 4>(a, grid, st);
+  else if (nw == 2) decode_kernel<T, D, 32, 2, SPLIT, true, 4>(a, grid, st);
+  else if (bn64) decode_kernel<T, D, 64, 4, SPLIT>(a, grid, st);
+  else decode_kernel<T, D, 32, 4, SPLIT>(a, grid, st);
 }
 
 template <class T, int D, int NQ>
@@ -276,7 +326,8 @@ void decode_stream(const gr_attn_args& a, int S, hipStream_t st) {
 // Decode-shape launch: Nq queries (any count) against N keys, non-causal, K in
 // [B, H, N, D]. Up to 4 queries: the streaming kernel (gr_flash_decode.h),
 // one workgroup per head and key part. More: the flash body with 32 queries
-// per wave, up to 4 waves, 64-key tiles (32 when N is not a multiple of 64).
+// per wave: up to 64 queries, four key groups per workgroup and 32-key tiles;
+// above, four waves and 64-key tiles (32 when N is not a multiple of 64).
 // S > 1 splits the keys over S workgroups per head (or query tile) and merges
 // their partials through the workspace.
 // Message for a workspace smaller than the key split needs: the caller's
@@ -308,17 +359,13 @@ int launch_decode(gr_attn_args a, int S, void* ws, size_t ws_bytes, bool fixed_w
     else decode_stream<T, D, 4>(a, S, st);
     int rc = gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_decode launch");
     if (rc != 0 || S == 1) return rc;
-    const long long threads = (long long)a.B * a.H * a.Nq * (D / 8);
-    hipLaunchKernelGGL((gr_attn_combine_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                       a.part_o, a.part_ml, static_cast<T*>(a.o), a.o_sb, a.o_sh, a.o_sn, a.B, a.H, a.Nq, S,
-                       a.scale_log2);
-    return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_decode combine launch");
+    return launch_combine<T, D>(a, S, st);
   }
   // fp16 with scale log2(e) > 1: Q as given (one wave per query tile, 32-key tiles)
   const bool unscaled = gr_is_same<T, _Float16>::value && a.scale_log2 > 1.0f;
   const int nw = unscaled ? 1 : a.Nq <= 32 ? 1 : a.Nq <= 64 ? 2 : 4;
   const long long nqt = (a.Nq + 32 * nw - 1) / (32 * nw);
-  const bool bn64 = !unscaled && a.N % 64 == 0;
+  const bool bn64 = nw == 4 && a.N % 64 == 0;
   const int bn = bn64 ? 64 : 32;
   const int tiles = a.N / bn;
   if (S < 1) S = 1;
@@ -340,19 +387,13 @@ int launch_decode(gr_attn_args a, int S, void* ws, size_t ws_bytes, bool fixed_w
       else decode_kernel<T, D, 32, 1, false, false>(a, grid, st);
     }
   } else if (S > 1) {
-    if (bn64) decode_nw<T, D, 64, true>(a, nw, grid, st);
-    else decode_nw<T, D, 32, true>(a, nw, grid, st);
+    decode_nw<T, D, true>(a, nw, bn64, grid, st);
   } else {
-    if (bn64) decode_nw<T, D, 64, false>(a, nw, grid, st);
-    else decode_nw<T, D, 32, false>(a, nw, grid, st);
+    decode_nw<T, D, false>(a, nw, bn64, grid, st);
   }
   int rc = gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_decode launch");
   if (rc != 0 || S == 1) return rc;
-  const long long threads = (long long)a.B * a.H * a.Nq * (D / 8);
-  hipLaunchKernelGGL((gr_attn_combine_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                     a.part_o, a.part_ml, static_cast<T*>(a.o), a.o_sb, a.o_sh, a.o_sn, a.B, a.H, a.Nq, S,
-                     a.scale_log2);
-  return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_decode combine launch");
+  return launch_combine<T, D>(a, S, st);
 }
 
 __global__ void gr_selftest_mfma32_kernel(const _Float16* A, const _Float16* B, float* Dm) {

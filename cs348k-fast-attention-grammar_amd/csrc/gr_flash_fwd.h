@@ -371,7 +371,7 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
   typedef gr_flash_lds<D, BN> L;
   static_assert(BN % 32 == 0 && D % 32 == 0, "tile shape");
   static_assert(!(SPLIT && (CAUSAL || PIPE)), "key split: non-causal, straight schedule");
-  static_assert(KG == 1 || (DIRECT && !PIPE && !SPLIT), "key groups: direct loads, straight schedule");
+  static_assert(KG == 1 || (DIRECT && !PIPE), "key groups: direct loads, straight schedule");
 
   const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / NT);   // key group
   const int tid = KG == 1 ? (int)threadIdx.x : (int)threadIdx.x - kg * NT;         // thread of the group

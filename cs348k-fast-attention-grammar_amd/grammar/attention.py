@@ -220,15 +220,24 @@ def flash_attention(q, k, v, *, causal: bool = False, scale: float | None = None
 
 
 def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256) -> int:
-    """Key parts per query tile for gr_attn_decode. Up to 4 queries (the
-    streaming kernel, 4 waves per workgroup): one workgroup per compute unit,
-    each part keeping at least 512 keys. More (the flash body): enough
-    workgroups for two per compute unit, each part keeping at least four
-    64-key tiles."""
+    """Key parts per query tile for gr_attn_decode, by the kernel that runs
+    (lines measured over B H 1-64, N 256-8192, both head dims):
+    1 query (streaming kernel): one workgroup per compute unit, parts of at
+    least 256 keys; up to 512 keys one launch is faster than two (D 64 N 512:
+    5.0 us against 7.2). 2 to 4 queries (the same kernel, more arithmetic per
+    key): two workgroups per compute unit and parts of 64 keys (B H 8, N 3104:
+    12.6 us at 32 parts, 20.6 at 6), one part up to 256 keys. 5 to 64 queries
+    (flash body, four key groups per workgroup): one workgroup per compute
+    unit, at most 16 parts of at least 256 keys (B H 16, N 8192: 13.2 us at 16
+    parts, 15.9 at 32). More: two workgroups per compute unit, each part
+    keeping at least four 64-key tiles."""
+    if Nq == 1:
+        return 1 if N <= 512 else max(1, min(-(-cu_count // (B * H)), N // 256, 32))
     if Nq <= 4:
-        return max(1, min(-(-cu_count // (B * H)), N // 512))
-    nw = 1 if Nq <= 32 else 2 if Nq <= 64 else 4
-    tiles_q = B * H * -(-Nq // (32 * nw))
+        return 1 if N <= 256 else max(1, min(-(-2 * cu_count // (B * H)), N // 64, 32))
+    if Nq <= 64:
+        return 1 if N <= 512 else max(1, min(cu_count // (B * H), N // 256, 16))
+    tiles_q = B * H * -(-Nq // 128)
     want = -(-2 * cu_count // tiles_q)
     return max(1, min(want, N // 256 if N >= 256 else 1))
 

@@ -1,0 +1,55 @@
+"""GPU parity of the decode launches' key groups (5 to 64 queries) and of the
+merge of their parts, against attention in float64 on the GPU.
+
+Bound: relative 2-norm at most the storage type's unit roundoff (2^-11 fp16,
+2^-8 bf16), as for the attention forward."""
+import math
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+CASES = [
+    # B, H, Nq, N, D, dtype, splits
+    (1, 2, 5, 32, 64, "fp16", 1),         # one key tile: three of four groups idle
+    (1, 2, 32, 96, 128, "bf16", 1),
+    (2, 3, 33, 224, 64, "bf16", 1),       # two waves, 31 queries past the end
+    (1, 3, 64, 1056, 128, "fp16", 4),     # four parts: lane groups merge a row each
+    (1, 5, 40, 1056, 64, "fp16", 5),      # five: a wave per row
+    (2, 1, 17, 3104, 128, "bf16", 16),
+    (1, 1, 9, 2144, 64, "bf16", 67),      # more parts than lanes in the merge
+    (1, 1, 3, 2144, 128, "fp16", 67),     # streaming kernel, the same merge
+    (1, 7, 1, 1024, 64, "bf16", 3),
+    (1, 2, 100, 544, 64, "fp16", 2),      # four waves, 32-key tiles, no groups
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
+def test_decode_groups_parity(case):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from grammar.attention import flash_attention_decode
+    B, H, Nq, N, D, dt, splits = case
+    print(f"[case] decode groups {case}", flush=True)
+    tdt = {"fp16": torch.float16, "bf16": torch.bfloat16}[dt]
+    g = torch.Generator("cpu").manual_seed(37)
+    q = torch.randn((B, H, Nq, D), generator=g)
+    # keys climb from part to part, so the parts and groups end with different bases
+    k = torch.randn((B, H, N + 64, D), generator=g) + (torch.arange(N + 64).float() * 2 / N).view(1, 1, -1, 1)
+    v = torch.randn((B, H, N + 64, D), generator=g)
+    q, k, v = (t.to(tdt).cuda() for t in (q, k, v))
+    k, v = k[:, :, :N], v[:, :, :N]                       # a cache with room for more
+    store = torch.full((B, H, Nq + 1, D), float("nan"), dtype=tdt, device="cuda")
+    o = flash_attention_decode(q, k, v, splits=splits, out=store[:, :, :Nq])
+    torch.cuda.synchronize()
+    assert torch.isnan(store[:, :, Nq].float()).all()
+    ref = torch.empty((B, H, Nq, D), dtype=torch.float64, device="cuda")
+    for b in range(B):
+        for h in range(H):
+            s = q[b, h].double() @ k[b, h].double().t().contiguous() / math.sqrt(D)
+            ref[b, h] = torch.softmax(s, dim=1) @ v[b, h].double()
+    err = float((o.double() - ref).norm() / ref.norm())
+    print(f"[parity] decode groups {case}: rel {err:.2e}", flush=True)
+    assert err <= (2.0 ** -11 if dt == "fp16" else 2.0 ** -8)
