@@ -17,8 +17,9 @@ import math
 from . import runtime as rt
 
 
-def _strides3(t, dims=(0, 1, 2)) -> "ctypes.Array":
-    return rt._ll3(*(int(t.stride(d)) for d in dims))
+def _strides3(t) -> "ctypes.Array":
+    st = t.stride()
+    return rt.strides3(st[0], st[1], st[2])
 
 
 def default_tiles(N: int, D: int, dtype: str | None = None, causal: bool = False) -> tuple:
@@ -35,6 +36,41 @@ def default_tiles(N: int, D: int, dtype: str | None = None, causal: bool = False
     return bm, bn
 
 
+def _fwd_args(q, k, v, lse, causal, scale, k_transposed, block_m, block_n, out, stream):
+    """(C arguments, out) of gr_attn_fwd, or (lse given) of gr_attn_fwd_train,
+    after checking the operands."""
+    import torch
+    dtype = q.dtype
+    for name, t in (("q", q), ("k", k), ("v", v)):
+        if not t.is_cuda:
+            raise ValueError(f"flash_attention_fwd: {name} must be a GPU tensor (no CPU path)")
+        if t.dtype != dtype:
+            raise ValueError("flash_attention_fwd: q, k, v must share a dtype")
+        if t.dim() != 4:
+            raise ValueError(f"flash_attention_fwd: {name} must be 4-D")
+    shape = q.shape
+    B, H, N, D = shape
+    if v.shape != shape:
+        raise ValueError(f"flash_attention_fwd: v shape {tuple(v.shape)} != q shape {tuple(shape)}")
+    want_k = (B, H, D, N) if k_transposed else shape
+    if k.shape != want_k:
+        raise ValueError(f"flash_attention_fwd: k shape {tuple(k.shape)} != {tuple(want_k)}")
+    if q.stride(3) != 1 or v.stride(3) != 1 or k.stride(3) != 1:
+        raise ValueError("flash_attention_fwd: innermost dimension must be contiguous")
+    if out is None:
+        out = torch.empty(shape, dtype=dtype, device=q.device)
+    elif out.shape != shape or out.dtype != dtype or out.stride(3) != 1:
+        raise ValueError("flash_attention_fwd: bad `out` tensor")
+    if scale is None:
+        scale = 1.0 / math.sqrt(D)
+    head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr())
+    if lse is not None:
+        head += (lse.data_ptr(),)
+    return head + (rt.dtype_code(dtype), B, H, N, D, _strides3(q), _strides3(k), _strides3(v), _strides3(out),
+                   int(bool(k_transposed)), int(bool(causal)), float(scale), int(block_m), int(block_n),
+                   rt._stream_ptr(stream)), out
+
+
 def bind_flash_attention(q, k, v, *, causal: bool = False, scale: float | None = None,
                          k_transposed: bool = False, block_m: int = 0, block_n: int = 0,
                          out=None, stream=None):
@@ -42,34 +78,8 @@ def bind_flash_attention(q, k, v, *, causal: bool = False, scale: float | None =
     gr_attn_fwd with the pre-packed C arguments (no per-call checks or
     allocation, for launch-bound loops such as a timing loop); out is the
     [B, H, N, D] result tensor it writes. Arguments as flash_attention_fwd."""
-    import torch
-    for name, t in (("q", q), ("k", k), ("v", v)):
-        if not t.is_cuda:
-            raise ValueError(f"flash_attention_fwd: {name} must be a GPU tensor (no CPU path)")
-        if t.dtype != q.dtype:
-            raise ValueError("flash_attention_fwd: q, k, v must share a dtype")
-        if t.dim() != 4:
-            raise ValueError(f"flash_attention_fwd: {name} must be 4-D")
-    B, H, N, D = q.shape
-    if tuple(v.shape) != (B, H, N, D):
-        raise ValueError(f"flash_attention_fwd: v shape {tuple(v.shape)} != q shape {tuple(q.shape)}")
-    want_k = (B, H, D, N) if k_transposed else (B, H, N, D)
-    if tuple(k.shape) != want_k:
-        raise ValueError(f"flash_attention_fwd: k shape {tuple(k.shape)} != {want_k}")
-    if q.stride(3) != 1 or v.stride(3) != 1 or k.stride(3) != 1:
-        raise ValueError("flash_attention_fwd: innermost dimension must be contiguous")
-    if out is None:
-        out = torch.empty((B, H, N, D), dtype=q.dtype, device=q.device)
-    elif tuple(out.shape) != (B, H, N, D) or out.dtype != q.dtype or out.stride(3) != 1:
-        raise ValueError("flash_attention_fwd: bad `out` tensor")
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
+    args, out = _fwd_args(q, k, v, None, causal, scale, k_transposed, block_m, block_n, out, stream)
     fn = rt.lib().gr_attn_fwd
-    args = (ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
-            ctypes.c_void_p(out.data_ptr()), rt.dtype_code(q.dtype), B, H, N, D,
-            _strides3(q), _strides3(k), _strides3(v), _strides3(out),
-            int(bool(k_transposed)), int(bool(causal)), float(scale), int(block_m), int(block_n),
-            rt._stream_ptr(stream))
     keep = (q, k, v, out)   # the tensors stay alive as long as the launcher
 
     def launch():
@@ -86,10 +96,20 @@ def flash_attention_fwd(q, k, v, *, causal: bool = False, scale: float | None = 
     q, v: [B, H, N, D]; k: [B, H, N, D], or [B, H, D, N] when k_transposed.
     All three share dtype (float16 or bfloat16) and live on the GPU. Returns a
     new [B, H, N, D] tensor (or writes `out`)."""
-    launch, out = bind_flash_attention(q, k, v, causal=causal, scale=scale, k_transposed=k_transposed,
-                                       block_m=block_m, block_n=block_n, out=out, stream=stream)
-    launch()
+    args, out = _fwd_args(q, k, v, None, causal, scale, k_transposed, block_m, block_n, out, stream)
+    rt.check(rt.lib().gr_attn_fwd(*args), "gr_attn_fwd")
     return out
+
+
+def _train_lse(q, lse):
+    """The [B, H, N] float32 row log-sum-exp to write: `lse`, checked, or a new one."""
+    import torch
+    shape = q.shape[:3]
+    if lse is None:
+        return torch.empty(shape, dtype=torch.float32, device=q.device)
+    if lse.shape != shape or lse.dtype != torch.float32 or not lse.is_contiguous():
+        raise ValueError("flash_attention_fwd_train: bad `lse` tensor")
+    return lse
 
 
 def bind_flash_attention_train(q, k, v, *, causal: bool = False, scale: float | None = None,
@@ -97,21 +117,11 @@ def bind_flash_attention_train(q, k, v, *, causal: bool = False, scale: float | 
     """bind_flash_attention for gr_attn_fwd_train: returns (launch, out, lse),
     launch() enqueueing the forward that also writes the row log-sum-exp of
     the scaled scores ([B, H, N] fp32, natural log). K in [B, H, N, D]."""
-    import torch
-    _, out = bind_flash_attention(q, k, v, causal=causal, scale=scale, block_m=block_m, block_n=block_n,
-                                  out=out, stream=stream)
-    B, H, N, D = q.shape
-    if lse is None:
-        lse = torch.empty((B, H, N), dtype=torch.float32, device=q.device)
-    elif tuple(lse.shape) != (B, H, N) or lse.dtype != torch.float32 or not lse.is_contiguous():
-        raise ValueError("flash_attention_fwd_train: bad `lse` tensor")
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
+    if q.dim() != 4:
+        raise ValueError("flash_attention_fwd: q must be 4-D")
+    lse = _train_lse(q, lse)
+    args, out = _fwd_args(q, k, v, lse, causal, scale, False, block_m, block_n, out, stream)
     fn = rt.lib().gr_attn_fwd_train
-    args = (ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
-            ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(lse.data_ptr()), rt.dtype_code(q.dtype), B, H, N, D,
-            _strides3(q), _strides3(k), _strides3(v), _strides3(out), 0, int(bool(causal)), float(scale),
-            int(block_m), int(block_n), rt._stream_ptr(stream))
     keep = (q, k, v, out, lse)
 
     def launch():
@@ -125,10 +135,44 @@ def flash_attention_fwd_train(q, k, v, *, causal: bool = False, scale: float | N
     """flash_attention_fwd that also returns the row log-sum-exp of the scaled
     scores ([B, H, N] fp32, natural log), kept for flash_attention_bwd.
     K in [B, H, N, D] layout. Returns (out, lse)."""
-    launch, out, lse = bind_flash_attention_train(q, k, v, causal=causal, scale=scale, block_m=block_m,
-                                                  block_n=block_n, out=out, lse=lse, stream=stream)
-    launch()
+    if q.dim() != 4:
+        raise ValueError("flash_attention_fwd: q must be 4-D")
+    lse = _train_lse(q, lse)
+    args, out = _fwd_args(q, k, v, lse, causal, scale, False, block_m, block_n, out, stream)
+    rt.check(rt.lib().gr_attn_fwd_train(*args), "gr_attn_fwd_train")
     return out, lse
+
+
+def _bwd_args(q, k, v, o, do, lse, causal, scale, workspace, grads, stream):
+    """(C arguments, gradients, workspace) of gr_attn_bwd after checking the
+    operands."""
+    import torch
+    shape, dtype = q.shape, q.dtype
+    B, H, N, D = shape
+    for name, t in (("q", q), ("k", k), ("v", v), ("o", o), ("do", do)):
+        if t.shape != shape or t.dtype != dtype or not t.is_cuda:
+            raise ValueError(f"flash_attention_bwd: {name} must match q ({tuple(shape)}, {dtype}, GPU)")
+        if not t.is_contiguous():
+            raise ValueError(f"flash_attention_bwd: {name} must be contiguous")
+    if lse.shape != (B, H, N) or lse.dtype != torch.float32 or not lse.is_contiguous():
+        raise ValueError("flash_attention_bwd: lse must be a contiguous [B, H, N] float32 tensor")
+    if scale is None:
+        scale = 1.0 / math.sqrt(D)
+    need = int(rt.lib().gr_attn_bwd_workspace(B, H, N, D))
+    if workspace is None:
+        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+    elif workspace.numel() * workspace.element_size() < need:
+        raise ValueError(f"flash_attention_bwd: workspace of {need} bytes needed")
+    if grads is None:
+        grads = (torch.empty_like(q), torch.empty_like(q), torch.empty_like(q))
+    else:
+        for t in grads:
+            if t.shape != shape or t.dtype != dtype or not t.is_contiguous():
+                raise ValueError("flash_attention_bwd: bad gradient tensor")
+    dq, dk, dv = grads
+    return (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr(),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), rt.dtype_code(dtype), B, H, N, D, _strides3(q),
+            int(bool(causal)), float(scale), workspace.data_ptr(), need, rt._stream_ptr(stream)), grads, workspace
 
 
 def bind_flash_attention_bwd(q, k, v, o, do, lse, *, causal: bool = False, scale: float | None = None,
@@ -138,35 +182,8 @@ def bind_flash_attention_bwd(q, k, v, o, do, lse, *, causal: bool = False, scale
     [B, H, N, D] fp16/bf16 GPU tensors of one dtype (the kernels take one
     stride set); lse: [B, H, N] float32 from the training forward; grads: an
     optional (dq, dk, dv) triple of such tensors to write."""
-    import torch
-    B, H, N, D = q.shape
-    for name, t in (("q", q), ("k", k), ("v", v), ("o", o), ("do", do)):
-        if tuple(t.shape) != (B, H, N, D) or t.dtype != q.dtype or not t.is_cuda:
-            raise ValueError(f"flash_attention_bwd: {name} must match q ({tuple(q.shape)}, {q.dtype}, GPU)")
-        if not t.is_contiguous():
-            raise ValueError(f"flash_attention_bwd: {name} must be contiguous")
-    if tuple(lse.shape) != (B, H, N) or lse.dtype != torch.float32 or not lse.is_contiguous():
-        raise ValueError("flash_attention_bwd: lse must be a contiguous [B, H, N] float32 tensor")
-    if scale is None:
-        scale = 1.0 / math.sqrt(D)
-    L = rt.lib()
-    need = int(L.gr_attn_bwd_workspace(B, H, N, D))
-    if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-    elif workspace.numel() * workspace.element_size() < need:
-        raise ValueError(f"flash_attention_bwd: workspace of {need} bytes needed")
-    if grads is None:
-        grads = (torch.empty_like(q), torch.empty_like(q), torch.empty_like(q))
-    for t in grads:
-        if tuple(t.shape) != (B, H, N, D) or t.dtype != q.dtype or not t.is_contiguous():
-            raise ValueError("flash_attention_bwd: bad gradient tensor")
-    dq, dk, dv = grads
-    fn = L.gr_attn_bwd
-    args = (ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
-            ctypes.c_void_p(o.data_ptr()), ctypes.c_void_p(do.data_ptr()), ctypes.c_void_p(lse.data_ptr()),
-            ctypes.c_void_p(dq.data_ptr()), ctypes.c_void_p(dk.data_ptr()), ctypes.c_void_p(dv.data_ptr()),
-            rt.dtype_code(q.dtype), B, H, N, D, _strides3(q), int(bool(causal)), float(scale),
-            ctypes.c_void_p(workspace.data_ptr()), need, rt._stream_ptr(stream))
+    args, grads, workspace = _bwd_args(q, k, v, o, do, lse, causal, scale, workspace, grads, stream)
+    fn = rt.lib().gr_attn_bwd
     keep = (q, k, v, o, do, lse, workspace, grads)
 
     def launch():
@@ -181,9 +198,8 @@ def flash_attention_bwd(q, k, v, o, do, lse, *, causal: bool = False, scale: flo
     lse (flash_attention_fwd_train). q, k, v, o, do: [B, H, N, D] fp16/bf16
     on the GPU (made contiguous here: the kernel takes one stride set)."""
     q, k, v, o, do, lse = (t.contiguous() for t in (q, k, v, o, do, lse))
-    launch, grads = bind_flash_attention_bwd(q, k, v, o, do, lse, causal=causal, scale=scale,
-                                             workspace=workspace, stream=stream)
-    launch()
+    args, grads, workspace = _bwd_args(q, k, v, o, do, lse, causal, scale, workspace, None, stream)
+    rt.check(rt.lib().gr_attn_bwd(*args), "gr_attn_bwd")
     return grads
 
 
@@ -253,39 +269,43 @@ def decode_splits_noalloc(B: int, H: int, Nq: int, N: int, D: int, cu_count: int
     return s
 
 
-def bind_flash_attention_decode(q, k, v, *, scale: float | None = None, splits: int = 0, out=None,
-                                workspace=None, stream=None):
-    """Validate once and return (launch, out) for gr_attn_decode, arguments
-    pre-packed (as bind_flash_attention); see flash_attention_decode."""
+def _decode_args(q, k, v, scale, splits, out, workspace, stream):
+    """(C arguments, out, workspace) of gr_attn_decode after checking the operands."""
     import torch
+    dtype = q.dtype
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not t.is_cuda:
             raise ValueError(f"flash_attention_decode: {name} must be a GPU tensor (no CPU path)")
-        if t.dtype != q.dtype or t.dim() != 4 or t.stride(3) != 1:
+        if t.dtype != dtype or t.dim() != 4 or t.stride(3) != 1:
             raise ValueError(f"flash_attention_decode: {name} must be 4-D, q's dtype, unit stride on D")
     B, H, Nq, D = q.shape
     N = k.shape[2]
-    if tuple(k.shape) != (B, H, N, D) or tuple(v.shape) != (B, H, N, D):
+    if k.shape != (B, H, N, D) or v.shape != (B, H, N, D):
         raise ValueError(f"flash_attention_decode: k {tuple(k.shape)} / v {tuple(v.shape)} do not match q {tuple(q.shape)}")
     if out is None:
-        out = torch.empty((B, H, Nq, D), dtype=q.dtype, device=q.device)
-    elif tuple(out.shape) != (B, H, Nq, D) or out.dtype != q.dtype or out.stride(3) != 1:
+        out = torch.empty((B, H, Nq, D), dtype=dtype, device=q.device)
+    elif out.shape != (B, H, Nq, D) or out.dtype != dtype or out.stride(3) != 1:
         raise ValueError("flash_attention_decode: bad `out` tensor")
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    L = rt.lib()
     if splits <= 0:
-        splits = decode_splits(B, H, Nq, N, rt.device_info(q.device.index or 0)["cu_count"])
-    need = int(L.gr_attn_decode_workspace(B, H, Nq, D, splits))
+        splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0))
+    need = int(rt.lib().gr_attn_decode_workspace(B, H, Nq, D, splits)) if splits > 1 else 0
     if need and workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     elif need and workspace.numel() * workspace.element_size() < need:
         raise ValueError(f"flash_attention_decode: workspace of {need} bytes needed")
-    fn = L.gr_attn_decode
-    args = (ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
-            ctypes.c_void_p(out.data_ptr()), rt.dtype_code(q.dtype), B, H, Nq, N, D,
+    return (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), rt.dtype_code(dtype), B, H, Nq, N, D,
             _strides3(q), _strides3(k), _strides3(v), _strides3(out), float(scale), int(splits),
-            ctypes.c_void_p(workspace.data_ptr() if need else None), need, rt._stream_ptr(stream))
+            workspace.data_ptr() if need else None, need, rt._stream_ptr(stream)), out, workspace
+
+
+def bind_flash_attention_decode(q, k, v, *, scale: float | None = None, splits: int = 0, out=None,
+                                workspace=None, stream=None):
+    """Validate once and return (launch, out) for gr_attn_decode, arguments
+    pre-packed (as bind_flash_attention); see flash_attention_decode."""
+    args, out, workspace = _decode_args(q, k, v, scale, splits, out, workspace, stream)
+    fn = rt.lib().gr_attn_decode
     keep = (q, k, v, out, workspace)
 
     def launch():
@@ -320,7 +340,7 @@ def bind_flash_attention_decode_noalloc(q, k, v, *, scale: float | None = None, 
         scale = 1.0 / math.sqrt(D)
     L = rt.lib()
     if splits <= 0:
-        splits = decode_splits_noalloc(B, H, Nq, N, D, rt.device_info(q.device.index or 0)["cu_count"])
+        splits = decode_splits_noalloc(B, H, Nq, N, D, rt.cu_count(q.device.index or 0))
     fn = L.gr_attn_decode_noalloc
     args = (ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
             ctypes.c_void_p(out.data_ptr()), rt.dtype_code(q.dtype), B, H, Nq, N, D,
@@ -340,9 +360,8 @@ def flash_attention_decode(q, k, v, *, scale: float | None = None, splits: int =
     q [B, H, Nq, D], k and v [B, H, N, D] (N a multiple of 32), fp16/bf16 on
     the GPU. splits = 0 picks the key split (decode_splits); the workspace
     it needs is allocated here unless given."""
-    launch, out = bind_flash_attention_decode(q, k, v, scale=scale, splits=splits, out=out,
-                                              workspace=workspace, stream=stream)
-    launch()
+    args, out, workspace = _decode_args(q, k, v, scale, splits, out, workspace, stream)
+    rt.check(rt.lib().gr_attn_decode(*args), "gr_attn_decode")
     return out
 
 

@@ -12,8 +12,6 @@ There is no CPU path: CPU tensors or a missing library raise.
 """
 from __future__ import annotations
 
-import ctypes
-
 from . import runtime as rt
 
 EPILOGUES = {"none": 0, "relu": 1, "silu": 2}
@@ -81,15 +79,15 @@ def gemm(a, b, *, epilogue: str = "none", alpha: float = 1.0, b_kmajor: bool = F
     if need:
         ws = rt.workspace(need, a.device, stream)
         rc = L.gr_gemm_ws(
-            ctypes.c_void_p(a.data_ptr()), ctypes.c_void_p(b.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-            dtype, za, M, N, K, rt._ll2(a_sb, a_sm), rt._ll2(b_sb, b_s), rt._ll2(c_sb, c_sm),
-            int(bool(b_kmajor)), EPILOGUES[epilogue], float(alpha), ctypes.c_void_p(ws.data_ptr()), need,
+            a.data_ptr(), b.data_ptr(), out.data_ptr(),
+            dtype, za, M, N, K, rt.strides2(a_sb, a_sm), rt.strides2(b_sb, b_s), rt.strides2(c_sb, c_sm),
+            int(bool(b_kmajor)), EPILOGUES[epilogue], float(alpha), ws.data_ptr(), need,
             rt._stream_ptr(stream))
         rt.check(rc, "gr_gemm_ws")
         return out
     rc = L.gr_gemm(
-        ctypes.c_void_p(a.data_ptr()), ctypes.c_void_p(b.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-        dtype, za, M, N, K, rt._ll2(a_sb, a_sm), rt._ll2(b_sb, b_s), rt._ll2(c_sb, c_sm),
+        a.data_ptr(), b.data_ptr(), out.data_ptr(),
+        dtype, za, M, N, K, rt.strides2(a_sb, a_sm), rt.strides2(b_sb, b_s), rt.strides2(c_sb, c_sm),
         int(bool(b_kmajor)), EPILOGUES[epilogue], float(alpha), int(block_m), int(block_n),
         rt._stream_ptr(stream))
     rt.check(rc, "gr_gemm")
@@ -123,14 +121,14 @@ def mlp_fwd(x, w1, w2, *, block_m: int = 0, block_n: int = 0, h=None, out=None, 
     if need:
         ws = rt.workspace(need, x.device, stream)
         rc = L.gr_mlp_fwd_ws(
-            ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(w1.data_ptr()), ctypes.c_void_p(w2.data_ptr()),
-            ctypes.c_void_p(h.data_ptr()), ctypes.c_void_p(out.data_ptr()), dtype,
-            M, D, F, ctypes.c_void_p(ws.data_ptr()), need, rt._stream_ptr(stream))
+            x.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+            h.data_ptr(), out.data_ptr(), dtype,
+            M, D, F, ws.data_ptr(), need, rt._stream_ptr(stream))
         rt.check(rc, "gr_mlp_fwd_ws")
         return out
     rc = L.gr_mlp_fwd(
-        ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(w1.data_ptr()), ctypes.c_void_p(w2.data_ptr()),
-        ctypes.c_void_p(h.data_ptr()), ctypes.c_void_p(out.data_ptr()), dtype,
+        x.data_ptr(), w1.data_ptr(), w2.data_ptr(),
+        h.data_ptr(), out.data_ptr(), dtype,
         M, D, F, int(block_m), int(block_n), rt._stream_ptr(stream))
     rt.check(rc, "gr_mlp_fwd")
     return out

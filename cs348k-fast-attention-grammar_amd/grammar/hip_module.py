@@ -131,7 +131,7 @@ class HipModule:
         self.code = code if code is not None else compile_cached(src)[0]
         self.module = rt.Module(self.code)
         self.kernels = [self.module.kernel(st["kernel"]) for st in self.plan["steps"]]
-        self._bound = None
+        self._template = None
 
     @property
     def dtype(self):
@@ -186,14 +186,58 @@ class HipModule:
             if not t.is_cuda:
                 raise ValueError(f"input {n} must be a GPU tensor (no CPU path)")
 
+    def _call_template(self):
+        """What every fn() call shares: (launch plan whose arguments are given
+        per run, the source of each argument, the inputs' shapes where a stage
+        reads them, elements of the intermediates' buffer). An argument's
+        source is ("in" | "out", index) or ("mid", byte offset): the
+        intermediates of a call live in one buffer, each at a multiple of 256
+        bytes."""
+        if self._template is None:
+            item = 4 if self.plan["dtype"] == "fp32" else 2
+            offsets, total = {}, 0
+            for name in self.plan["intermediates"]:
+                offsets[name] = total * item
+                n = 1
+                for d in self.plan["tensors"][name]:
+                    n *= int(d)
+                total += -(-n * item // 256) * 256 // item
+            where = {n: ("in", i) for i, n in enumerate(self.inputs)}
+            where.update({n: ("out", i) for i, n in enumerate(self.plan["outputs"])})
+            where.update({n: ("mid", off) for n, off in offsets.items()})
+            steps = [(k, st["grid"], st["block"], st["lds"], [0] * len(st["args"]))
+                     for st, k in zip(self.plan["steps"], self.kernels)]
+            names = [a for st in self.plan["steps"] for a in st["args"]]
+            read = set(names)
+            shapes = [tuple(self.plan["tensors"][n]) if n in read else None for n in self.inputs]
+            self._template = (rt.Plan(steps), [where[a] for a in names], shapes, total)
+        return self._template
+
     def fn(self, *inputs):
         """Run the module on `inputs` (sorted-name order) and return the output
-        (or a tuple of outputs)."""
+        (or a tuple of outputs). Outputs and intermediates start NaN-filled
+        (allocate()); the intermediates share one buffer and one fill."""
+        import torch
         self._check_inputs(inputs)
-        tensors = dict(zip(self.inputs, inputs))
-        tensors.update(self.allocate(inputs[0].device))
-        self.bind(tensors).run()
-        outs = [tensors[o] for o in self.plan["outputs"]]
+        if self.plan.get("check"):                   # a checking build also binds its findings buffer
+            tensors = dict(zip(self.inputs, inputs))
+            tensors.update(self.allocate(inputs[0].device))
+            self.bind(tensors).run()
+            outs = [tensors[o] for o in self.plan["outputs"]]
+            return outs[0] if len(outs) == 1 else tuple(outs)
+        plan, sources, shapes, total = self._call_template()
+        dtype, device = self.dtype, inputs[0].device
+        for n, t, shape in zip(self.inputs, inputs, shapes):
+            if shape is not None and (t.shape != shape or t.dtype != dtype or not t.is_contiguous()):
+                raise ValueError(f"tensor {n}: need contiguous {self.plan['tensors'][n]} {dtype}, "
+                                 f"got {tuple(t.shape)} {t.dtype}")
+        nan = float("nan")
+        outs = [torch.empty(tuple(self.plan["tensors"][o]), dtype=dtype, device=device).fill_(nan)
+                for o in self.plan["outputs"]]
+        mid = torch.empty(total, dtype=dtype, device=device).fill_(nan) if total else None
+        base = {"in": [t.data_ptr() for t in inputs], "out": [t.data_ptr() for t in outs]}
+        mid_ptr = mid.data_ptr() if total else 0
+        plan.run_args([mid_ptr + i if kind == "mid" else base[kind][i] for kind, i in sources])
         return outs[0] if len(outs) == 1 else tuple(outs)
 
     __call__ = fn

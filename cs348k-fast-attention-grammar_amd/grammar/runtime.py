@@ -11,6 +11,7 @@ loading fails loudly otherwise -- there is no CPU fallback on this path.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -46,6 +47,19 @@ _ll3 = ctypes.c_longlong * 3
 _ll2 = ctypes.c_longlong * 2
 
 
+@functools.lru_cache(maxsize=1024)
+def strides3(s0: int, s1: int, s2: int):
+    """A C array of three strides. Shared by every call with the same values
+    (the library only reads it)."""
+    return _ll3(s0, s1, s2)
+
+
+@functools.lru_cache(maxsize=1024)
+def strides2(s0: int, s1: int):
+    """strides3 for two strides."""
+    return _ll2(s0, s1)
+
+
 def lib() -> ctypes.CDLL:
     """The loaded library (raises if it was never built)."""
     global _lib
@@ -79,6 +93,7 @@ def lib() -> ctypes.CDLL:
         L.gr_plan_create.argtypes = [i32, ctypes.POINTER(vp)]
         L.gr_plan_set_step.argtypes = [vp, i32, vp, _u32x3, _u32x3, ctypes.c_uint32, u64p, i32]
         L.gr_plan_run.argtypes = [vp, vp]
+        L.gr_plan_run_args.argtypes = [vp, vp, u64p, i32]
         L.gr_plan_free.argtypes = [vp]
         L.gr_plan_free.restype = None
         L.gr_plan_time.argtypes = [vp, vp, i32, i32, i32, ctypes.POINTER(ctypes.c_float)]
@@ -118,7 +133,7 @@ EXPORTED = (
     "gr_plan_set_step", "gr_plan_run", "gr_plan_free", "gr_plan_time", "gr_attn_fwd",
     "gr_selftest_mfma32", "gr_gemm", "gr_mlp_fwd", "gr_attn_decode_workspace", "gr_attn_decode",
     "gr_attn_fwd_train", "gr_attn_bwd_workspace", "gr_attn_bwd", "gr_attn_decode_noalloc",
-    "gr_gemm_workspace", "gr_gemm_ws", "gr_mlp_fwd_workspace", "gr_mlp_fwd_ws",
+    "gr_plan_run_args", "gr_gemm_workspace", "gr_gemm_ws", "gr_mlp_fwd_workspace", "gr_mlp_fwd_ws",
 )
 
 # Bytes of the per-device scratch array behind gr_attn_decode_noalloc (GR_DECODE_SCRATCH_BYTES).
@@ -144,6 +159,12 @@ def device_info(device: int = 0) -> dict:
     check(lib().gr_device_info(device, out), "gr_device_info")
     return {"cu_count": out[0], "lds_per_block": out[1], "wave_size": out[2],
             "clock_khz": out[3], "l2_bytes": out[4]}
+
+
+@functools.lru_cache(maxsize=64)
+def cu_count(device: int = 0) -> int:
+    """Compute units of a device (read once per device)."""
+    return device_info(device)["cu_count"]
 
 
 def compile_source(src: str, name: str = "gr_module.hip", options: list[str] | None = None) -> bytes:
@@ -205,11 +226,13 @@ class Module:
             pass
 
 
-def _stream_ptr(stream) -> ctypes.c_void_p:
+def _stream_ptr(stream) -> int:
+    """The hipStream_t of `stream` (a torch stream or a raw handle), or of the
+    current stream of the current device if None."""
     if stream is None:
         import torch
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream))
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
 def workspace(nbytes: int, device, stream=None):
@@ -242,6 +265,13 @@ class Plan:
     def run(self, stream=None) -> None:
         check(lib().gr_plan_run(self.handle, _stream_ptr(stream)), "gr_plan_run")
 
+    def run_args(self, args, stream=None) -> None:
+        """Run with this call's u64 arguments (the steps' one after another)
+        instead of the bound ones."""
+        n = len(args)
+        check(lib().gr_plan_run_args(self.handle, _stream_ptr(stream), (ctypes.c_uint64 * n)(*args), n),
+              "gr_plan_run_args")
+
     def time(self, warmup: int, iters: int, mode: int = GR_TIME_BATCH, stream=None) -> float:
         ms = ctypes.c_float()
         check(lib().gr_plan_time(self.handle, _stream_ptr(stream), warmup, iters, mode, ctypes.byref(ms)),
@@ -260,12 +290,16 @@ class Plan:
             pass
 
 
+_DTYPE_CODES: dict = {}
+
+
 def dtype_code(torch_dtype) -> int:
-    import torch
-    if torch_dtype == torch.float16:
-        return GR_F16
-    if torch_dtype == torch.bfloat16:
-        return GR_BF16
-    if torch_dtype == torch.float32:
-        return GR_F32
-    raise ValueError(f"unsupported dtype {torch_dtype}")
+    code = _DTYPE_CODES.get(torch_dtype)
+    if code is None:
+        import torch
+        codes = {torch.float16: GR_F16, torch.bfloat16: GR_BF16, torch.float32: GR_F32}
+        if torch_dtype not in codes:
+            raise ValueError(f"unsupported dtype {torch_dtype}")
+        _DTYPE_CODES.update(codes)
+        code = codes[torch_dtype]
+    return code
