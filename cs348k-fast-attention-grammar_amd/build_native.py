@@ -46,7 +46,10 @@ COMMON = [
 # accumulators stay in VGPRs, and the dK/dV accumulators, pinned to AGPRs by
 # inline assembly, need no copies either (the d = 64 kernels are faster with
 # the heuristics).
-EXTRA = {"gr_attn_bwd128.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# The fp32 attention forward reads its score accumulators on the vector ALU the
+# same way.
+EXTRA = {"gr_attn_bwd128.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+         "gr_attn_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _sources() -> list[str]:

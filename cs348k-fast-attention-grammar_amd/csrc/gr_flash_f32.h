@@ -39,12 +39,16 @@ struct gr_flash32_lds {
   static constexpr int BYTES = (O_FLOATS + NW * 32 * 2) * 4;
 };
 
-// nkb: 32-key blocks per wave when the chunk length is only known at run time
-// (the library launches: nkb = N / (32 NW PARTS)); 0 takes BN / 32.
-template <int D, int BN, int NW, bool KT_LAYOUT, int PARTS>
+// blocks: the call's 32-key blocks, N / 32, shared out over the NW PARTS waves
+// in consecutive runs that differ by at most one (the library launches; a wave
+// may get none); 0: BN / 32 blocks each (rendered stages).
+// ONE: every wave has exactly one block (no branch, loop or rescale: 6.3 ->
+// 5.9 us at D 64, N 512, one head).
+// WIDE: 64-bit lane addresses for V and K^T (row strides of 2^27 elements and
+// more), else a wave-uniform row pointer plus a 32-bit lane offset.
+template <int D, int BN, int NW, bool KT_LAYOUT, int PARTS, bool WIDE = false, bool ONE = false>
 __device__ __forceinline__ void gr_flash32_fwd_body(const gr_attn_args& a, char* lds, float* ws_o, float* ws_ml,
-                                                    int nkb = 0) {
-  const int KB = nkb > 0 ? nkb : BN / 32;   // 32-key blocks per wave
+                                                    int blocks = 0) {
   constexpr int DB = D / 32;       // 32-wide head-dim blocks of O^T
   constexpr int DG = D / 8;        // groups of 8 d (4 MFMAs of 2)
   constexpr int SL = D / NW;       // head dims each wave merges
@@ -54,16 +58,19 @@ __device__ __forceinline__ void gr_flash32_fwd_body(const gr_attn_args& a, char*
   const int g = lane >> 5, l32 = lane & 31;
   const int lead = a.B * a.H;
   const int nqb = a.N / 32;
-  const int wg = blockIdx.x;
+  const int wg = gr_xcd_remap_any((int)blockIdx.x, (int)gridDim.x);
   const int bh = wg / (nqb * PARTS);
   const int rem = wg % (nqb * PARTS);
-  const int qblk = rem / PARTS, part = rem % PARTS;
+  const int part = rem / nqb, qblk = rem % nqb;        // an XCD's workgroups share a part's keys
   const int b = bh / a.H, h = bh % a.H;
   const float* Qp = (const float*)a.q + b * a.q_sb + h * a.q_sh;
   const float* Kp = (const float*)a.k + b * a.k_sb + h * a.k_sh;
   const float* Vp = (const float*)a.v + b * a.v_sb + h * a.v_sh;
   float* Op = (float*)a.o + b * a.o_sb + h * a.o_sh;
-  const int q0 = qblk * 32, k0 = (part * NW + wave) * 32 * KB;
+  const int q0 = qblk * 32;
+  const int chunk = part * NW + __builtin_amdgcn_readfirstlane(wave);
+  const int b0 = blocks > 0 ? blocks * chunk / (NW * PARTS) : chunk * (BN / 32);                 // first key block
+  const int nb = blocks > 0 ? blocks * (chunk + 1) / (NW * PARTS) - b0 : BN / 32;                // their count
   const float c = a.scale_log2;
 
   gr_f32x4 qf[DG];
@@ -71,27 +78,44 @@ __device__ __forceinline__ void gr_flash32_fwd_body(const gr_attn_args& a, char*
   for (int dg = 0; dg < DG; ++dg)
     qf[dg] = *reinterpret_cast<const gr_f32x4*>(Qp + (long long)(q0 + l32) * a.q_sn + 8 * dg + 4 * g);
 
-  // operands of one 32-key block: K (MFMA A of the scores) and V (MFMA A of P V).
-  // Each lane keeps one base pointer per operand; the rest of every address
-  // is wave-uniform (scalar arithmetic when the strides are run-time values).
-  const float* const k_lane = KT_LAYOUT ? Kp + (long long)(4 * g) * a.k_sn + l32 : Kp + (long long)l32 * a.k_sn + 4 * g;
-  const float* const v_lane = Vp + (long long)(4 * g) * a.v_sn + l32;
-  auto load_k = [&](int kr, gr_f32x4 (&kf)[DG]) {
-#pragma unroll
-    for (int dg = 0; dg < DG; ++dg) {
-      if constexpr (KT_LAYOUT) {
-#pragma unroll
-        for (int t = 0; t < 4; ++t) kf[dg][t] = k_lane[(long long)(8 * dg + t) * a.k_sn + kr];
-      } else {
-        kf[dg] = *reinterpret_cast<const gr_f32x4*>(k_lane + (long long)kr * a.k_sn + 8 * dg);
+  // Operands of one 32-key block: K (MFMA A of the scores) and V (MFMA A of P
+  // V). V and K^T are read down a column of the tile, one row per load: a
+  // wave-uniform row pointer stepped by the stride (two scalar adds) plus the
+  // lane's 32-bit offset, made opaque per block so that it stays 32 bits wide
+  // (as hoisted 64-bit lane addresses the loads cost a vector add each, as
+  // products by run-time strides more scalar time than the MFMAs).
+  const unsigned int v_off = (unsigned int)(4 * g * a.v_sn + l32) * 4u, k_off = (unsigned int)(4 * g * a.k_sn + l32) * 4u;
+  const float* const k_lane = Kp + (long long)l32 * a.k_sn + 4 * g;          // natural K: the lane's key row
+  auto column = [&](const float* base, unsigned int off, long long g_elems) {   // base + off, as the load wants it
+    struct ptr {
+      const char* row;
+      unsigned int off;
+      __device__ __forceinline__ float at(int bytes) const {
+        return *reinterpret_cast<const float*>(row + off + bytes);
       }
+    };
+    if constexpr (WIDE) return ptr{reinterpret_cast<const char*>(base + g_elems), 0u};
+    asm volatile("" : "+v"(off));
+    return ptr{reinterpret_cast<const char*>(base), off};
+  };
+  // a block's K, group dg of 8 d at a time, from p (K^T, stepped) or kp
+  auto k_column = [&](int kr) { return column(Kp + kr, k_off, 4 * g * a.k_sn + l32); };
+  auto load_k = [&](auto& p, int kr, int dg, gr_f32x4 (&kf)[DG]) {
+    if constexpr (KT_LAYOUT) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        kf[dg][t] = p.at(0);
+        p.row += a.k_sn * 4 * (t == 3 ? 5 : 1);
+      }
+    } else {
+      kf[dg] = *reinterpret_cast<const gr_f32x4*>(k_lane + (long long)kr * a.k_sn + 8 * dg);
     }
   };
-  auto load_v = [&](int kr, float (&vf)[DB][16]) {
+  // its V, row t at a time
+  auto load_v = [&](auto& p, int t, float (&vf)[DB][16]) {
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int t = 0; t < 16; ++t) vf[db][t] = v_lane[(long long)(kr + 8 * (t >> 2) + (t & 3)) * a.v_sn + 32 * db];
+    for (int db = 0; db < DB; ++db) vf[db][t] = p.at(128 * db);
+    p.row += a.v_sn * 4 * ((t & 3) == 3 ? 5 : 1);
   };
 
   gr_f32x16 o[DB];
@@ -100,49 +124,78 @@ __device__ __forceinline__ void gr_flash32_fwd_body(const gr_attn_args& a, char*
   float m = -GR_INF, l = 0.f;
   gr_f32x4 kf[DG];
   float vf[DB][16];
-  load_k(k0, kf);
-  load_v(k0, vf);
-#pragma unroll 1
-  for (int kb = 0; kb < KB; ++kb) {
-    gr_f32x4 kn[DG];
-    float vn[DB][16];
-    if (kb + 1 < KB) {
-      load_k(k0 + 32 * (kb + 1), kn);
-      load_v(k0 + 32 * (kb + 1), vn);
-    }
-    gr_f32x16 s = (gr_f32x16)(0.f);
+  gr_f32x16 s;
+  // One 32-key block, its K in kf: S^T = K Q^T (s[r]: key 8 (r / 4) + 4 g + r
+  // % 4, query q0 + l32), the online softmax, O^T += V^T P^T. One buffer each
+  // for K and V: V's rows are loaded between the score MFMAs and (NEXT) the
+  // K of block `next` between the P V MFMAs, in the order of their use, so
+  // that every load has 2,048 (d = 64) or 4,096 cycles of MFMAs to land behind
+  // and its address arithmetic issues under them (all loads ahead of the MFMAs
+  // took D 128, one block per wave, from 8.8 to 9.5 us). HOLD pins that order;
+  // the compiler's own is the better one only for a single block of natural K
+  // at D 128 (9.8 -> 9.5 us; at D 64 5.9 -> 7.4).
+  constexpr bool HOLD = !(ONE && D == 128 && !KT_LAYOUT);
+  auto block = [&](int kr, int next, auto next_tag) {
+    constexpr bool NEXT = decltype(next_tag)::value;
+    auto vp = column(Vp + (long long)kr * a.v_sn, v_off, 4 * g * a.v_sn + l32);
+    s = (gr_f32x16)(0.f);
 #pragma unroll
-    for (int dg = 0; dg < DG; ++dg)
+    for (int dg = 0; dg < DG; ++dg) {
+#pragma unroll
+      for (int t = dg * 16 / DG; t < (dg + 1) * 16 / DG; ++t) load_v(vp, t, vf);
 #pragma unroll
       for (int t = 0; t < 4; ++t) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[dg][t], qf[dg][t], s, 0, 0, 0);
-    // s[r]: key 8 (r / 4) + 4 g + r % 4 of the block, query q0 + l32
+      if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
+    }
     float mt = -GR_INF;
 #pragma unroll
     for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[r]);
     mt = fmaxf(mt, gr_xor32(mt));
     const float mn = fmaxf(m, mt);
-    const float alpha = gr_exp2((m - mn) * c);   // m = -inf -> 0
-    l *= alpha;
+    if constexpr (ONE) {                           // nothing before it
+      m = mt;
+    } else if (gr_any(mn > m)) {                   // else every factor is 1
+      const float alpha = gr_exp2((m - mn) * c);   // m = -inf -> 0
+      l *= alpha;
 #pragma unroll
-    for (int db = 0; db < DB; ++db) o[db] *= alpha;
-    m = mn;
+      for (int db = 0; db < DB; ++db) o[db] *= alpha;
+      m = mn;
+    }
     const float mc = m * c;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       s[r] = gr_exp2(fmaf(s[r], c, -mc));
       l += s[r];
     }
+    auto kp = k_column(next);
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+    for (int t = 0; t < 16; ++t) {
+      if constexpr (NEXT) {
 #pragma unroll
-      for (int t = 0; t < 16; ++t) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db][t], s[t], o[db], 0, 0, 0);
-    if (kb + 1 < KB) {
+        for (int dg = t * DG / 16; dg < (t + 1) * DG / 16; ++dg) load_k(kp, next, dg, kf);
+      }
 #pragma unroll
-      for (int dg = 0; dg < DG; ++dg) kf[dg] = kn[dg];
+      for (int db = 0; db < DB; ++db) o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[db][t], s[t], o[db], 0, 0, 0);
+      if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  if (ONE || nb > 0) {
+    {
+      auto kp = k_column(32 * b0);
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int t = 0; t < 16; ++t) vf[db][t] = vn[db][t];
+      for (int dg = 0; dg < DG; ++dg) load_k(kp, 32 * b0, dg, kf);
+    }
+    // The last block: from K^T it loads its own K again, from natural K it is a
+    // copy of the body without that load (16-byte loads that are not wanted cost
+    // more than the copy's join, which waits for K).
+    if (ONE || (blocks == 0 && BN == 32)) {
+      block(32 * b0, 0, gr_ic<0>{});
+    } else {
+      constexpr int COPY = KT_LAYOUT ? 0 : 1;
+#pragma unroll 1
+      for (int i = 0; i < nb - COPY; ++i)
+        block(32 * (b0 + i), 32 * (b0 + gr_imin(i + 1, nb - 1)), gr_ic<1>{});
+      if constexpr (COPY == 1) block(32 * (b0 + nb - 1), 0, gr_ic<0>{});
     }
   }
   l += gr_xor32(l);

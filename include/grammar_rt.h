@@ -118,14 +118,16 @@ int gr_plan_time(gr_plan* p, void* stream, int warmup, int iters, int mode, floa
  *  throughout on the fp32 matrix cores): non-causal only, N a multiple of 32,
  *  block_m and block_n ignored (a workgroup owns 32 queries and splits its
  *  keys over its waves); not for gr_attn_fwd_train. When B * H * N / 32 query
- *  blocks would leave CUs idle (N a multiple of 256, at most 128 blocks), the
- *  keys of a query block are also split over 2, 4 or 8 workgroups and a
- *  second launch merges their partials, which sit in a workspace the library
- *  allocates once per (device, stream) and grows on demand: at most
- *  256 * 32 * (D + 2) * 4 bytes (4.3 MB at D = 128), since a split launch has
- *  at most 256 workgroups of 32 queries. A grown buffer is kept until the
- *  process ends, and on the per-thread default stream each host thread keeps
- *  its own. Call once on a stream before capturing such calls into a graph.
+ *  blocks would leave CUs idle, the keys of a query block are also split over
+ *  2, 4 or 8 workgroups (the library picks by D, N, the query blocks and the
+ *  CU count) and a second launch merges their partials, which sit in a
+ *  workspace the library allocates once per (device, stream) and keeps until
+ *  the process ends: 4.3 MB, for a split launch has at most 256 workgroups of
+ *  32 queries. On the per-thread default stream each host thread has its own.
+ *  Without memory for it the call runs unsplit. Under capture only N a
+ *  multiple of 256 with at most 128 query blocks is split, over the most of 8,
+ *  4 or 2 workgroups that divide N / 128; call once on a stream before
+ *  capturing such calls into a graph.
  *  Q, V, O: [B, H, N, D] with strides {batch, head, seq} in elements
  *  (unit stride along D). K: [B, H, N, D] if k_transposed == 0, else KT
  *  [B, H, D, N] whose k_strides = {batch, head, d} (unit stride along N).

@@ -1,0 +1,99 @@
+"""GPU parity of the fp32 attention forward where its 32-key blocks share out
+unevenly over the waves and workgroups of a query block, against float64.
+
+Bound per element: scores are float32 sums of D products, so |ds| <= (D + 4)
+2^-24 scale sum |q k|; a weight's relative error is 2 |ds| plus the exponentials'
+2^-22, one more 2^-22 for each of the N / 32 rescales; O sums N products. With w
+the weights, |error| <= (2 (2 max |ds| + (N / 32 + 2) 2^-22) + (N + 8) 2^-24)
+sum w |v|."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+U = 2.0 ** -24
+
+
+def _cuda():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch.device("cuda:0")
+
+
+def _inputs(heads, N, D, dev, seed=41):
+    g = torch.Generator("cpu").manual_seed(seed)
+    # keys that grow along the sequence: the running maximum moves block by block
+    ramp = torch.linspace(0.2, 2.0, N).view(1, 1, N, 1)
+    q, k, v = (torch.randn((1, heads, N, D), generator=g) for _ in range(3))
+    return q.to(dev), (k * ramp).to(dev), v.to(dev)
+
+
+def _check(got, q, k, v, what):
+    N, D = q.shape[2:]
+    scale = D ** -0.5
+    q64, k64, v64 = (t.double() for t in (q, k, v))
+    w = torch.softmax(scale * (q64 @ k64.transpose(2, 3).contiguous()), -1)
+    ds = (D + 4) * U * scale * (q64.abs() @ k64.abs().transpose(2, 3).contiguous()).amax(-1, keepdim=True)
+    bound = (2 * (2 * ds + (N // 32 + 2) * 2.0 ** -22) + (N + 8) * U) * (w @ v64.abs())
+    err = (got.double() - w @ v64).abs()
+    print(f"[parity] fp32 blocks {what}: max {float(err.max()):.2e}", flush=True)
+    assert bool((err <= bound).all())
+
+
+CASES = [
+    # heads, N: 32-key blocks per wave
+    (1, 32),       # one wave has a block, three have none
+    (3, 96),       # three have one
+    (1, 128),      # one each
+    (2, 160),      # two and one; from here on split over workgroups
+    (1, 512),      # one each in four parts
+    (4, 320),
+    (1, 1056),     # 33 blocks over 32 waves
+    (3, 1184),     # two parts, four and five
+    (40, 224),     # more workgroups than compute units
+]
+
+
+@pytest.mark.parametrize("kt", [False, True], ids=["natural", "kt"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("heads,N", CASES)
+def test_fp32_blocks_parity(heads, N, D, kt):
+    dev = _cuda()
+    from grammar.attention import flash_attention_fwd
+    print(f"[case] fp32 blocks heads={heads} N={N} D={D} kt={kt}", flush=True)
+    q, k, v = _inputs(heads, N, D, dev)
+    out = torch.full((1, heads, N + 1, D + 8), float("nan"), device=dev)
+    kk = k.transpose(2, 3).contiguous() if kt else k
+    flash_attention_fwd(q, kk, v, k_transposed=kt, out=out[:, :, :N, :D])
+    again = flash_attention_fwd(q, kk, v, k_transposed=kt)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, :, :N, :D], again)
+    assert torch.isnan(out[:, :, N:]).all() and torch.isnan(out[..., D:]).all()
+    _check(again, q, k, v, (heads, N, D, kt))
+
+
+@pytest.mark.parametrize("kt", [False, True], ids=["natural", "kt"])
+def test_fp32_blocks_wide_row_strides(kt):
+    """Rows of V and K^T 2^27 elements apart: past the 32-bit lane offsets."""
+    dev = _cuda()
+    from grammar.attention import flash_attention_fwd
+    N = D = 64
+    row = 1 << 27
+    need = (63 * row + 2 * D) * 4
+    if torch.cuda.mem_get_info(dev)[0] < need + (4 << 30):
+        pytest.skip("needs 34 GB of device memory")
+    print(f"[case] fp32 wide row strides kt={kt}", flush=True)
+    q, k, v = _inputs(1, N, D, dev)
+    buf = torch.empty(need // 4, device=dev)
+    vw = buf.as_strided((1, 1, N, D), (row, row, row, 1))
+    vw.copy_(v)
+    kk = k
+    if kt:
+        kk = buf.as_strided((1, 1, D, N), (row, row, row, 1), D)
+        kk.copy_(k.transpose(2, 3))
+    got = flash_attention_fwd(q, kk, vw, k_transposed=kt)
+    torch.cuda.synchronize()
+    _check(got, q, k, v, ("wide", kt))
+    del buf, vw, kk
+    torch.cuda.empty_cache()
