@@ -23,11 +23,11 @@ namespace {
 // N 2048, D 128 278 us (124 TFLOP/s; with equal power-of-two shares of the
 // keys, K and V double-buffered and 64-bit row products per load it was 406),
 // 8 heads D 64 72 us (was 94); below that by the longest wave.
-template <int D, bool KT, int PARTS, bool WIDE, bool ONE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1)))
+template <int D, int NW, bool KT, int PARTS, bool WIDE, int ONE>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1)))
 void gr_flash32_kernel(gr_attn_args a, int blocks, float* ws_o, float* ws_ml) {
   extern __shared__ __attribute__((aligned(16))) char gr_lds[];
-  gr_flash32_fwd_body<D, 32, 4, KT, PARTS, WIDE, ONE>(a, gr_lds, ws_o, ws_ml, blocks);
+  gr_flash32_fwd_body<D, 32, NW, KT, PARTS, WIDE, ONE>(a, gr_lds, ws_o, ws_ml, blocks);
 }
 
 template <int D, int PARTS>
@@ -88,12 +88,22 @@ bool capturing(hipStream_t st) {
 template <int D, bool KT, int PARTS, bool WIDE = false>
 int launch_parts(const gr_attn_args& a, long long nblk, float* ws_o, float* ws_ml, hipStream_t st) {
   const dim3 grid((unsigned)(nblk * PARTS));
-  if (!WIDE && a.N / 32 == 4 * PARTS)
-    hipLaunchKernelGGL((gr_flash32_kernel<D, KT, PARTS, false, true>), grid, dim3(256), (gr_flash32_lds<D, 4>::BYTES),
-                       st, a, a.N / 32, ws_o, ws_ml);
+  constexpr int LDS = gr_flash32_lds<D, 4>::BYTES;
+  const int blocks = a.N / 32;
+  // one and two blocks: as many waves (5 heads, N 32, D 128: 7.2 us, 7.8 with
+  // three idle waves in the merge)
+  if (!WIDE && PARTS == 1 && blocks == 1)
+    hipLaunchKernelGGL((gr_flash32_kernel<D, 1, KT, 1, false, 1>), grid, dim3(64), (gr_flash32_lds<D, 1>::BYTES), st, a,
+                       blocks, ws_o, ws_ml);
+  else if (!WIDE && PARTS == 1 && blocks == 2)
+    hipLaunchKernelGGL((gr_flash32_kernel<D, 2, KT, 1, false, 1>), grid, dim3(128), (gr_flash32_lds<D, 2>::BYTES), st, a,
+                       blocks, ws_o, ws_ml);
+  else if (!WIDE && blocks == 4 * PARTS)
+    hipLaunchKernelGGL((gr_flash32_kernel<D, 4, KT, PARTS, false, 1>), grid, dim3(256), LDS, st, a, blocks, ws_o, ws_ml);
+  else if (!WIDE && blocks < 4 * PARTS)
+    hipLaunchKernelGGL((gr_flash32_kernel<D, 4, KT, PARTS, false, 2>), grid, dim3(256), LDS, st, a, blocks, ws_o, ws_ml);
   else
-    hipLaunchKernelGGL((gr_flash32_kernel<D, KT, PARTS, WIDE, false>), grid, dim3(256), (gr_flash32_lds<D, 4>::BYTES),
-                       st, a, a.N / 32, ws_o, ws_ml);
+    hipLaunchKernelGGL((gr_flash32_kernel<D, 4, KT, PARTS, WIDE, 0>), grid, dim3(256), LDS, st, a, blocks, ws_o, ws_ml);
   return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_fwd fp32 launch");
 }
 

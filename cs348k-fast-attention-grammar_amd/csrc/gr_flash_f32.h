@@ -42,11 +42,11 @@ struct gr_flash32_lds {
 // blocks: the call's 32-key blocks, N / 32, shared out over the NW PARTS waves
 // in consecutive runs that differ by at most one (the library launches; a wave
 // may get none); 0: BN / 32 blocks each (rendered stages).
-// ONE: every wave has exactly one block (no branch, loop or rescale: 6.3 ->
-// 5.9 us at D 64, N 512, one head).
+// ONE: 1: every wave has exactly one block (no branch, loop or rescale: 6.3 ->
+// 5.9 us at D 64, N 512, one head); 2: at most one.
 // WIDE: 64-bit lane addresses for V and K^T (row strides of 2^27 elements and
 // more), else a wave-uniform row pointer plus a 32-bit lane offset.
-template <int D, int BN, int NW, bool KT_LAYOUT, int PARTS, bool WIDE = false, bool ONE = false>
+template <int D, int BN, int NW, bool KT_LAYOUT, int PARTS, bool WIDE = false, int ONE = 0>
 __device__ __forceinline__ void gr_flash32_fwd_body(const gr_attn_args& a, char* lds, float* ws_o, float* ws_ml,
                                                     int blocks = 0) {
   constexpr int DB = D / 32;       // 32-wide head-dim blocks of O^T
@@ -179,7 +179,7 @@ __device__ __forceinline__ void gr_flash32_fwd_body(const gr_attn_args& a, char*
       if constexpr (HOLD) __builtin_amdgcn_sched_barrier(0);
     }
   };
-  if (ONE || nb > 0) {
+  if (ONE == 1 || nb > 0) {
     {
       auto kp = k_column(32 * b0);
 #pragma unroll

@@ -43,8 +43,9 @@ def _check(got, q, k, v, what):
 
 CASES = [
     # heads, N: 32-key blocks per wave
-    (1, 32),       # one wave has a block, three have none
-    (3, 96),       # three have one
+    (1, 32),       # one wave, one block
+    (2, 64),       # two waves
+    (3, 96),       # three of four waves have one
     (1, 128),      # one each
     (2, 160),      # two and one; from here on split over workgroups
     (1, 512),      # one each in four parts
