@@ -242,15 +242,22 @@ def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256) -> int:
     least 256 keys; up to 512 keys one launch is faster than two (D 64 N 512:
     5.0 us against 7.2). 2 to 4 queries (the same kernel, more arithmetic per
     key): two workgroups per compute unit and parts of 64 keys (B H 8, N 3104:
-    12.6 us at 32 parts, 20.6 at 6), one part up to 256 keys. 5 to 64 queries
+    12.6 us at 32 parts, 20.6 at 6), one part up to 256 keys. With heads for more
+    than half the compute units both are bound by memory and take one workgroup
+    per compute unit and parts of 512 keys (B H 180, N 832: 17.1 us in one
+    part, 19.3 in two; B H 182, N 3072, 2 queries: 59 in two, 68 in three),
+    except 2 to 4 queries below 1,024 keys and one head per unit. 5 to 64 queries
     (flash body, four key groups per workgroup): one workgroup per compute
     unit, at most 16 parts of at least 256 keys (B H 16, N 8192: 13.2 us at 16
     parts, 15.9 at 32). More: two workgroups per compute unit, each part
     keeping at least four 64-key tiles."""
+    heads = B * H
+    if Nq <= 4 and 2 * heads > cu_count and (Nq == 1 or N >= 1024 or heads >= cu_count):
+        return max(1, min(-(-cu_count // heads), N // 512))
     if Nq == 1:
-        return 1 if N <= 512 else max(1, min(-(-cu_count // (B * H)), N // 256, 32))
+        return 1 if N <= 512 else max(1, min(-(-cu_count // heads), N // 256, 32))
     if Nq <= 4:
-        return 1 if N <= 256 else max(1, min(-(-2 * cu_count // (B * H)), N // 64, 32))
+        return 1 if N <= 256 else max(1, min(-(-2 * cu_count // heads), N // 64, 32))
     if Nq <= 64:
         return 1 if N <= 512 else max(1, min(cu_count // (B * H), N // 256, 16))
     tiles_q = B * H * -(-Nq // 128)
