@@ -78,6 +78,9 @@ constexpr AttnShape kShapes128[] = {
     {2, 4, 32, 1.297, 1.333, 3.92, 1.37}, {4, 2, 64, 1.989, 1.990, 2.50, 1.81}, {2, 1, 64, 1.287, 0.704, 3.50, 0.67},
     {4, 1, 64, 1.129, 1.000, 3.05, 0.83}, {8, 1, 64, 1.665, 1.733, 3.73, 0.27},
 };
+// 128 x 128 at D = 64 (compiled for whole query tiles), non-causal: 17 heads at
+// N 2432 43.2 us, 45.1 on 128 x 64 and 46.4 on 64 x 64
+constexpr AttnShape kShape128x128 = {4, 1, 128, 1.26, 1.03, 3.1, 0.75};
 // the two-wave bodies at 256 x 64 (gr_flash_w2.h, gr_flash_w2h.h)
 constexpr AttnShape kShapeW2 = {8, 1, 64, 0.653, 0.961, 0.46, 1.19};
 constexpr AttnShape kShapeW2h = {8, 1, 64, 1.080, 1.585, 2.61, 0.71};
@@ -87,10 +90,17 @@ AttnShape pick_shape(int D, bool causal, bool two_wave, long long heads, int N) 
   const int cus = gr::cu_count() > 0 ? gr::cu_count() : 256;
   AttnShape best = {0, 0, 0, 0, 0, 0, 0};
   double best_t = 1e30;
-  auto consider = [&](const AttnShape& s) {
+  auto consider = [&](AttnShape s) {
     const int bm = 32 * s.nw;
     const double w = (double)heads * ((N + bm - 1) / bm), iters = ((N + s.bn - 1) / s.bn + s.kg - 1) / s.kg;
     double mean = iters, rounds = (double)(long long)((w + cus - 1) / cus);
+    // 64 x 64 at D = 64, non-causal: a CU's first two workgroups of two waves
+    // share SIMDs (9 heads, N 2432: 44.9 us for 342 workgroups), and a fifth
+    // waits for LDS (26 heads, N 2944: 91 us for 1,196)
+    if (!causal && D == 64 && s.nw == 2 && s.kg == 1) {
+      if (w > cus) s.lat = 1.08;
+      if (w > 4. * cus) s.thr = 0.36;
+    }
     if (causal) {              // longest first, so a part round costs about a quarter
       mean *= 0.5 + 0.5 * bm / (N > bm ? N : bm);
       rounds = w <= cus ? 1. : w / cus + 0.25;
@@ -106,6 +116,7 @@ AttnShape pick_shape(int D, bool causal, bool two_wave, long long heads, int N) 
   if (D == 64)
     for (const AttnShape& s : kShapes64)
       if (!(two_wave && s.nw == 8)) consider(s);
+  if (D == 64 && !causal && N % 256 == 128) consider(kShape128x128);
   if (D == 128)
     for (const AttnShape& s : kShapes128)
       if (!(two_wave && s.nw == 8)) consider(s);
@@ -128,6 +139,8 @@ int dispatch_tiles(const gr_attn_args& a, int bm, int bn, hipStream_t st) {
     const AttnShape s = pick_shape(D, CAUSAL, two_wave, (long long)a.B * a.H, a.N);
     if (s.kg > 1)
       return gr::launch_flash_groups(a, gr_is_same<T, _Float16>::value ? GR_F16 : GR_BF16, D, CAUSAL, KT, s.nw, s.kg, st);
+    if constexpr (D == 64 && !CAUSAL)
+      if (s.bn == 128) return launch_flash<T, D, 128, 4, 1, CAUSAL, KT>(a, st);
     if (s.nw == 2) return launch_flash<T, D, 64, 2, 1, CAUSAL, KT>(a, st, true);
     if (s.nw == 4) return launch_flash<T, D, 64, 4, 1, CAUSAL, KT>(a, st, true);
     if (a.N % 256 != 0) return launch_flash<T, D, 64, 8, 1, CAUSAL, KT>(a, st, true);

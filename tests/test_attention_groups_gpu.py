@@ -43,6 +43,7 @@ CASES = [
     (2, 2, 512, 64, "bf16", False, True),
     (1, 1, 2048, 64, "fp16", True, False),    # 1 wave x 8 groups
     (1, 2, 1344, 64, "bf16", False, False),
+    (1, 15, 2432, 64, "bf16", False, False),   # 128-query tiles of 128 keys
     (1, 16, 1024, 64, "fp16", False, False),  # 2 waves x 2 groups
     (1, 32, 320, 64, "bf16", True, True),
     (1, 12, 1408, 64, "bf16", False, False),  # 4 waves x 2 groups
