@@ -70,14 +70,23 @@ struct gr_attn_args {
 // register-transposing variants always take the max pass): after the first
 // key tile P is computed with the current base and no max pass; only when
 // some p overflowed the P type (the row max grew by more than ~16 powers of
-// two in fp16) is the tile redone with the max pass and a rescale. Q is
-// pre-scaled by scale log2(e) and the score MFMAs start from -base, so p is
-// one exp2 of the accumulator. The score MFMAs of a tile then need not all
-// finish before its first exponentials, and ~100 VALU instructions per
-// 128-key tile and wave drop out.
+// two in fp16) or a row sum passed GR_FLASH_SUM_MAX (bf16) is the tile redone
+// with the max pass and a rescale. In fp16 Q is pre-scaled by scale log2(e) and
+// the score MFMAs start from -base, so p is one exp2 of the accumulator. The
+// score MFMAs of a tile then need not all finish before its first exponentials,
+// and ~100 VALU instructions per 128-key tile and wave drop out.
 #ifndef GR_FLASH_OPT
 #define GR_FLASH_OPT 1
 #endif
+
+// Largest row sum of a tile (per lane) whose P is kept with the current base;
+// above it the tile is redone with the base at the true max. bf16's P reaches
+// 2^127, but a base is brought to another one's (a later tile's, group's or key
+// part's) by a factor of at least 2^-126 or 0, v_exp_f32 having no subnormal
+// results: a p of 2^127 would be lost in full with a base 127 below the row's
+// max, and sums of such p overflow. From 2^60 what a factor of 0 drops is below
+// 2^-66 of the row. (fp16's P overflows at 2^16, long before.)
+#define GR_FLASH_SUM_MAX 0x1p60f
 
 template <int V> struct gr_ic { static constexpr int value = V; };
 template <bool C, class X, class Y> struct gr_cond { typedef X type; };
@@ -738,8 +747,8 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
         // bf16: Q is not pre-scaled (its rounding would cost 2^-8), one
         // multiply-add per score instead
         // P of the whole tile with the current base; the max pass runs only on
-        // the first tile and when some p overflowed (then the base moves to
-        // the true max and P is recomputed).
+        // the first tile and when a row sum passed GR_FLASH_SUM_MAX or a p
+        // overflowed (then the base moves to the true max and P is recomputed).
         vec8 pt[KB][2][QB];
         float lt[QB];
         auto make_p = [&](const float (&nmc)[QB]) {
@@ -779,7 +788,7 @@ __device__ __forceinline__ void gr_flash_fwd_body(const gr_attn_args& a, char* l
           make_p(nmc);
           bool bad = false;
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) bad |= !(lt[qb] <= 3.0e38f);   // an inf (or NaN) p
+          for (int qb = 0; qb < QB; ++qb) bad |= !(lt[qb] <= GR_FLASH_SUM_MAX);   // too far above the base
           ok = !gr_any(bad);
         }
         if (!ok) {

@@ -33,8 +33,8 @@
 //
 // Softmax: the base m of a row is the max of its first tile's scaled scores;
 // p = 2^(s c - m). A step with a row sum past the P type's range (a row max
-// that grew by about 2^16 for fp16; an fp32 overflow for bf16) is redone on a
-// slow path that moves the base and rescales the accumulators.
+// that grew by about 2^16 for fp16) or, for bf16, past GR_FLASH_SUM_MAX is
+// redone on a slow path that moves the base and rescales the accumulators.
 //
 // Hazards the compiler does not see through inline assembly are kept apart
 // by construction: every score register is read by the vector unit at least
@@ -58,7 +58,7 @@ template <>
 struct gr_w2h_ops<__bf16> {
   static constexpr const char* mfma = "v_mfma_f32_32x32x16_bf16";
   static constexpr const char* pack = "v_cvt_pk_bf16_f32";
-  static constexpr float sum_max = 3.0e38f;     // only an fp32 overflow
+  static constexpr float sum_max = GR_FLASH_SUM_MAX;
 };
 
 // The vector work of one slot on score x: t = 2^(x c + nm), the previous
@@ -359,7 +359,7 @@ __device__ __forceinline__ void gr_flash_w2h_body(const gr_attn_args& a, char* l
     // the last score's p joins the sum; the step's row sums to fp32 lsum
     asm volatile("v_add_f32 %0, %0, %1" : "+v"(la) : "v"(tB));
     float ltq = la;
-    // a p (or a row sum) past the P type's range reads as > sum_max (or NaN)
+    // a p (or a row sum) past the bound reads as > sum_max (or NaN)
     if (__builtin_expect(gr_any(!(ltq <= OP::sum_max)), 0)) {
       asm volatile(GR_W2H_GUARD : "+v"(S_next[0]), "+v"(S_next[1]), "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]));
       // Slow path: the base moves to the true (scaled) row max of tile j,
