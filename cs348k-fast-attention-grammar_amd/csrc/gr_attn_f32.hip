@@ -56,6 +56,7 @@ struct F32Workspace {
 };
 std::mutex g_f32_ws_lock;
 std::vector<F32Workspace> g_f32_ws;
+thread_local int t_fail_workspaces = 0;   // gr_selftest_f32_no_workspace: lookups still to fail
 
 // The caller holds g_f32_ws_lock, and keeps it over the launches that use the
 // buffer: another thread's split call on the same stream then queues behind
@@ -65,13 +66,19 @@ int f32_workspace(hipStream_t st, void** out) {
   int rc = gr::hip_check(hipGetDevice(&dev), GR_E_RUNTIME, "gr_attn_fwd: hipGetDevice");
   if (rc) return rc;
   const std::thread::id thread = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
-  for (auto& e : g_f32_ws)
-    if (e.dev == dev && e.st == st && e.thread == thread) {
-      *out = e.p;
-      return GR_OK;
-    }
+  size_t bytes = kF32WorkspaceBytes;
+  if (t_fail_workspaces > 0) {
+    --t_fail_workspaces;
+    bytes = (size_t)1 << 60;              // more than any device has
+  } else {
+    for (auto& e : g_f32_ws)
+      if (e.dev == dev && e.st == st && e.thread == thread) {
+        *out = e.p;
+        return GR_OK;
+      }
+  }
   void* p = nullptr;
-  rc = gr::hip_check(hipMalloc(&p, kF32WorkspaceBytes), GR_E_RUNTIME, "gr_attn_fwd: fp32 key-split workspace");
+  rc = gr::hip_check(hipMalloc(&p, bytes), GR_E_RUNTIME, "gr_attn_fwd: fp32 key-split workspace");
   if (rc) return rc;
   g_f32_ws.push_back({dev, st, thread, p});
   *out = p;
@@ -185,4 +192,10 @@ int gr::attn_fwd_f32(const gr_attn_args& a, int D, bool causal, bool k_transpose
   if (D == 64) return k_transposed ? launch_flash32<64, true>(a, st) : launch_flash32<64, false>(a, st);
   if (D == 128) return k_transposed ? launch_flash32<128, true>(a, st) : launch_flash32<128, false>(a, st);
   return gr::fail(GR_E_ARG, "gr_attn_fwd: head dim %d unsupported (64 or 128)", D);
+}
+
+extern "C" int gr_selftest_f32_no_workspace(int lookups) {
+  if (lookups < 0) return gr::fail(GR_E_ARG, "gr_selftest_f32_no_workspace: negative count");
+  t_fail_workspaces = lookups;
+  return GR_OK;
 }

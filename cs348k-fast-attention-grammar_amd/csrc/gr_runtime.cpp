@@ -21,6 +21,7 @@ namespace gr {
 
 int hip_check(hipError_t e, int code, const char* what) {
   if (e == hipSuccess) return GR_OK;
+  (void)hipGetLastError();   // reported here: a later launch's hipGetLastError() must not find it
   return fail(code, "%s: %s (%d)", what, hipGetErrorString(e), (int)e);
 }
 

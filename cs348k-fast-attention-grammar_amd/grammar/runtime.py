@@ -100,6 +100,7 @@ def lib() -> ctypes.CDLL:
         L.gr_attn_fwd.argtypes = [vp, vp, vp, vp, i32, i32, i32, i32, i32, _ll3, _ll3, _ll3, _ll3,
                                   i32, i32, ctypes.c_float, i32, i32, vp]
         L.gr_selftest_mfma32.argtypes = [vp, vp, vp, vp]
+        L.gr_selftest_f32_no_workspace.argtypes = [i32]
         L.gr_gemm.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, _ll2, _ll2, _ll2, i32, i32,
                               ctypes.c_float, i32, i32, vp]
         L.gr_gemm_workspace.argtypes = [i32, i32, i32, i32, i32]
@@ -134,6 +135,7 @@ EXPORTED = (
     "gr_selftest_mfma32", "gr_gemm", "gr_mlp_fwd", "gr_attn_decode_workspace", "gr_attn_decode",
     "gr_attn_fwd_train", "gr_attn_bwd_workspace", "gr_attn_bwd", "gr_attn_decode_noalloc",
     "gr_plan_run_args", "gr_gemm_workspace", "gr_gemm_ws", "gr_mlp_fwd_workspace", "gr_mlp_fwd_ws",
+    "gr_selftest_f32_no_workspace",
 )
 
 # Bytes of the per-device scratch array behind gr_attn_decode_noalloc (GR_DECODE_SCRATCH_BYTES).

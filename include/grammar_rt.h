@@ -279,6 +279,11 @@ int gr_mlp_fwd_ws(const void* x, const void* w1, const void* w2, void* h, void* 
  * fp32 out, all row-major device buffers). */
 int gr_selftest_mfma32(const void* a, const void* b, float* d, void* stream);
 
+/* Self-test of the fp32 attention's unsplit path: the calling thread's next
+ * `lookups` key-split workspaces fail to allocate (each asks the device for
+ * more memory than it has), whether or not the stream has one already. */
+int gr_selftest_f32_no_workspace(int lookups);
+
 #ifdef __cplusplus
 }
 #endif

@@ -98,3 +98,25 @@ def test_fp32_blocks_wide_row_strides(kt):
     _check(got, q, k, v, ("wide", kt))
     del buf, vw, kk
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("heads,N,D", [(1, 512, 64), (4, 320, 64), (3, 1184, 128)])
+def test_fp32_split_without_memory_for_its_workspace(heads, N, D):
+    """A key split whose workspace cannot be allocated runs unsplit and reports
+    success, and the failed allocation is not found by a later call."""
+    dev = _cuda()
+    from grammar import runtime as rt
+    from grammar.attention import flash_attention_fwd
+    print(f"[case] fp32 without a workspace heads={heads} N={N} D={D}", flush=True)
+    q, k, v = _inputs(heads, N, D, dev)
+    split = flash_attention_fwd(q, k, v)
+    rt.check(rt.lib().gr_selftest_f32_no_workspace(1))
+    try:
+        whole = flash_attention_fwd(q, k, v)
+        assert "workspace" in rt.last_error()            # the hook was reached
+    finally:
+        rt.check(rt.lib().gr_selftest_f32_no_workspace(0))
+    again = flash_attention_fwd(q, k, v)
+    torch.cuda.synchronize()
+    _check(whole, q, k, v, ("no workspace", heads, N, D))
+    assert torch.equal(split, again)
