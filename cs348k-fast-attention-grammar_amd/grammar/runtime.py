@@ -237,6 +237,17 @@ def _stream_ptr(stream) -> int:
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
+def torch_stream(stream, device):
+    """The torch stream of `stream` (a torch stream or a raw handle)."""
+    import torch
+    if hasattr(stream, "cuda_stream"):
+        return stream
+    handle = int(stream)
+    if handle == 0:                  # ExternalStream(0) would be a new stream of torch's pool
+        return torch.cuda.default_stream(device)
+    return torch.cuda.ExternalStream(handle, device=device)
+
+
 def workspace(nbytes: int, device, stream=None):
     """`nbytes` of device memory for a launch on `stream` (the current stream
     if None), allocated for that stream: once dropped it is only reused by
@@ -244,9 +255,7 @@ def workspace(nbytes: int, device, stream=None):
     import torch
     if stream is None:
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    if not hasattr(stream, "cuda_stream"):
-        stream = torch.cuda.ExternalStream(int(stream), device=device)
-    with torch.cuda.stream(stream):
+    with torch.cuda.stream(torch_stream(stream, device)):
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
