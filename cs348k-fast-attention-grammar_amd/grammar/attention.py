@@ -160,7 +160,7 @@ def _bwd_args(q, k, v, o, do, lse, causal, scale, workspace, grads, stream):
         scale = 1.0 / math.sqrt(D)
     need = int(rt.lib().gr_attn_bwd_workspace(B, H, N, D))
     if workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        workspace = rt.workspace(need, q.device, stream)
     elif workspace.numel() * workspace.element_size() < need:
         raise ValueError(f"flash_attention_bwd: workspace of {need} bytes needed")
     if grads is None:
@@ -197,7 +197,7 @@ def flash_attention_bwd(q, k, v, o, do, lse, *, causal: bool = False, scale: flo
     """dQ, dK, dV of sum(O * dO) for the attention forward that produced o and
     lse (flash_attention_fwd_train). q, k, v, o, do: [B, H, N, D] fp16/bf16
     on the GPU (made contiguous here: the kernel takes one stride set)."""
-    q, k, v, o, do, lse = (t.contiguous() for t in (q, k, v, o, do, lse))
+    q, k, v, o, do, lse = (rt.contiguous(t, stream) for t in (q, k, v, o, do, lse))
     args, grads, workspace = _bwd_args(q, k, v, o, do, lse, causal, scale, workspace, None, stream)
     rt.check(rt.lib().gr_attn_bwd(*args), "gr_attn_bwd")
     return grads
@@ -299,7 +299,7 @@ def _decode_args(q, k, v, scale, splits, out, workspace, stream):
         splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0))
     need = int(rt.lib().gr_attn_decode_workspace(B, H, Nq, D, splits)) if splits > 1 else 0
     if need and workspace is None:
-        workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        workspace = rt.workspace(need, q.device, stream)
     elif need and workspace.numel() * workspace.element_size() < need:
         raise ValueError(f"flash_attention_decode: workspace of {need} bytes needed")
     return (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), rt.dtype_code(dtype), B, H, Nq, N, D,

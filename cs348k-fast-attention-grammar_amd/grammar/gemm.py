@@ -109,7 +109,7 @@ def mlp_fwd(x, w1, w2, *, block_m: int = 0, block_n: int = 0, h=None, out=None, 
     if tuple(w1.shape) != (D, F) or tuple(w2.shape) != (F, D):
         raise ValueError(f"mlp_fwd: shapes x{tuple(x.shape)} w1{tuple(w1.shape)} w2{tuple(w2.shape)}")
     if h is None:
-        h = torch.empty((M, F), dtype=x.dtype, device=x.device)
+        h = rt.empty((M, F), x.dtype, x.device, stream)
     if out is None:
         out = torch.empty((M, D), dtype=x.dtype, device=x.device)
     for name, t, shp in (("h", h, (M, F)), ("out", out, (M, D))):

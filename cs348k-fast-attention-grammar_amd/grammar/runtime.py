@@ -248,15 +248,30 @@ def torch_stream(stream, device):
     return torch.cuda.ExternalStream(handle, device=device)
 
 
-def workspace(nbytes: int, device, stream=None):
-    """`nbytes` of device memory for a launch on `stream` (the current stream
-    if None), allocated for that stream: once dropped it is only reused by
-    work queued there later."""
+def empty(shape, dtype, device, stream=None):
+    """torch.empty for a launch on `stream` (the current stream if None),
+    allocated for that stream: once dropped it is only reused by work queued
+    there later."""
     import torch
     if stream is None:
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return torch.empty(shape, dtype=dtype, device=device)
     with torch.cuda.stream(torch_stream(stream, device)):
-        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return torch.empty(shape, dtype=dtype, device=device)
+
+
+def workspace(nbytes: int, device, stream=None):
+    """`nbytes` of device memory, as empty()."""
+    import torch
+    return empty(nbytes, torch.uint8, device, stream)
+
+
+def contiguous(t, stream=None):
+    """t.contiguous() for a launch on `stream`: a copy is made there."""
+    import torch
+    if stream is None or t.is_contiguous():
+        return t.contiguous()
+    with torch.cuda.stream(torch_stream(stream, t.device)):
+        return t.contiguous()
 
 
 class Plan:
