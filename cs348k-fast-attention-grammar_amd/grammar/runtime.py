@@ -248,6 +248,9 @@ def torch_stream(stream, device):
     return torch.cuda.ExternalStream(handle, device=device)
 
 
+_STREAM_PER_THREAD = 2               # hipStreamPerThread
+
+
 def empty(shape, dtype, device, stream=None):
     """torch.empty for a launch on `stream` (the current stream if None),
     allocated for that stream: once dropped it is only reused by work queued
@@ -255,7 +258,15 @@ def empty(shape, dtype, device, stream=None):
     import torch
     if stream is None:
         return torch.empty(shape, dtype=dtype, device=device)
-    with torch.cuda.stream(torch_stream(stream, device)):
+    s = torch_stream(stream, device)
+    if s.cuda_stream == _STREAM_PER_THREAD:
+        # One handle for another stream in every host thread: memory kept by
+        # handle would pass between them. The current stream's, ordered by events.
+        t = torch.empty(shape, dtype=dtype, device=device)
+        s.wait_stream(torch.cuda.current_stream(device))
+        t.record_stream(s)
+        return t
+    with torch.cuda.stream(s):
         return torch.empty(shape, dtype=dtype, device=device)
 
 
@@ -270,8 +281,9 @@ def contiguous(t, stream=None):
     import torch
     if stream is None or t.is_contiguous():
         return t.contiguous()
+    c = empty(t.shape, t.dtype, t.device, stream)
     with torch.cuda.stream(torch_stream(stream, t.device)):
-        return t.contiguous()
+        return c.copy_(t)
 
 
 class Plan:

@@ -87,3 +87,42 @@ def test_scratch_goes_back_to_the_launch_stream(call, raw):
     assert _free_bytes(side.cuda_stream) - before[1] >= size
     for g, w in zip(got if isinstance(got, tuple) else (got,), want if isinstance(want, tuple) else (want,)):
         assert torch.equal(g, w)
+
+
+def test_per_thread_streams_do_not_share_memory():
+    """hipStreamPerThread is one handle for another stream in every host
+    thread: what one thread drops with work in flight, no other thread gets."""
+    dev = _cuda()
+    import threading
+    from grammar import runtime as rt
+    from grammar.gemm import gemm
+    size, handle = 48 << 20, 2
+    a, b = torch.randn(24, 4096, device=dev).half(), torch.randn(4096, 1376, device=dev).half()
+    want = gemm(a, b)
+    torch.cuda.synchronize()
+    got, dropped, checked = {}, threading.Event(), threading.Event()
+
+    def first():
+        ws = rt.workspace(size, dev, handle)
+        with torch.cuda.stream(rt.torch_stream(handle, dev)):
+            torch.cuda._sleep(50_000_000)
+        got["first"] = ws.data_ptr()
+        del ws
+        got["busy"] = not rt.torch_stream(handle, dev).query()
+        dropped.set()
+        checked.wait(30)
+        got["c"] = gemm(a, b, stream=handle)
+        rt.torch_stream(handle, dev).synchronize()
+
+    def second():
+        dropped.wait(30)
+        got["second"] = rt.workspace(size, dev, handle).data_ptr()
+        checked.set()
+
+    threads = [threading.Thread(target=f) for f in (first, second)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert got["busy"] and got["second"] != got["first"]
+    assert torch.equal(got["c"], want)
