@@ -235,7 +235,7 @@ def flash_attention(q, k, v, *, causal: bool = False, scale: float | None = None
     return _FLASH_FN.apply(q, k, v, causal, scale)
 
 
-def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256) -> int:
+def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256, *, groups: bool = True) -> int:
     """Key parts per query tile for gr_attn_decode, by the kernel that runs
     (lines measured over B H 1-64, N 256-8192, both head dims):
     1 query (streaming kernel): one workgroup per compute unit, parts of at
@@ -249,8 +249,10 @@ def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256) -> int:
     except 2 to 4 queries below 1,024 keys and one head per unit. 5 to 64 queries
     (flash body, four key groups per workgroup): one workgroup per compute
     unit, at most 16 parts of at least 256 keys (B H 16, N 8192: 13.2 us at 16
-    parts, 15.9 at 32). More: two workgroups per compute unit, each part
-    keeping at least four 64-key tiles."""
+    parts, 15.9 at 32). More, and the kernel without key groups (groups=False:
+    fp16 with scale log2(e) > 1): two workgroups per compute unit, each part
+    keeping at least four 64-key tiles (without groups B H 129, N 8192, D 64: 52
+    us in four parts, 153 in one)."""
     heads = B * H
     if Nq <= 4 and 2 * heads > cu_count and (Nq == 1 or N >= 1024 or heads >= cu_count):
         return max(1, min(-(-cu_count // heads), N // 512))
@@ -258,19 +260,25 @@ def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256) -> int:
         return 1 if N <= 512 else max(1, min(-(-cu_count // heads), N // 256, 32))
     if Nq <= 4:
         return 1 if N <= 256 else max(1, min(-(-2 * cu_count // heads), N // 64, 32))
-    if Nq <= 64:
+    if Nq <= 64 and groups:
         return 1 if N <= 512 else max(1, min(cu_count // (B * H), N // 256, 16))
     tiles_q = B * H * -(-Nq // 128)
     want = -(-2 * cu_count // tiles_q)
     return max(1, min(want, N // 256 if N >= 256 else 1))
 
 
-def decode_splits_noalloc(B: int, H: int, Nq: int, N: int, D: int, cu_count: int = 256) -> int:
+def _key_groups(dtype, scale) -> bool:
+    """Whether decode launches of 5 to 64 queries have key groups: not where fp16
+    keeps Q as given (launch_decode's rule)."""
+    return rt.dtype_code(dtype) != rt.GR_F16 or float(scale) * math.log2(math.e) <= 1.0
+
+
+def decode_splits_noalloc(B: int, H: int, Nq: int, N: int, D: int, cu_count: int = 256, *, groups: bool = True) -> int:
     """decode_splits, lowered until the key parts' partials fit the library's
     scratch array (rt.DECODE_SCRATCH_BYTES), which gr_attn_decode_noalloc
     cannot grow. One part needs no scratch."""
     L = rt.lib()
-    s = decode_splits(B, H, Nq, N, cu_count)
+    s = decode_splits(B, H, Nq, N, cu_count, groups=groups)
     while s > 1 and int(L.gr_attn_decode_workspace(B, H, Nq, D, s)) > rt.DECODE_SCRATCH_BYTES:
         s -= 1
     return s
@@ -296,7 +304,7 @@ def _decode_args(q, k, v, scale, splits, out, workspace, stream):
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     if splits <= 0:
-        splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0))
+        splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0), groups=_key_groups(dtype, scale))
     need = int(rt.lib().gr_attn_decode_workspace(B, H, Nq, D, splits)) if splits > 1 else 0
     if need and workspace is None:
         workspace = rt.workspace(need, q.device, stream)
@@ -347,7 +355,8 @@ def bind_flash_attention_decode_noalloc(q, k, v, *, scale: float | None = None, 
         scale = 1.0 / math.sqrt(D)
     L = rt.lib()
     if splits <= 0:
-        splits = decode_splits_noalloc(B, H, Nq, N, D, rt.cu_count(q.device.index or 0))
+        splits = decode_splits_noalloc(B, H, Nq, N, D, rt.cu_count(q.device.index or 0),
+                                       groups=_key_groups(q.dtype, scale))
     fn = L.gr_attn_decode_noalloc
     args = (ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()), ctypes.c_void_p(v.data_ptr()),
             ctypes.c_void_p(out.data_ptr()), rt.dtype_code(q.dtype), B, H, Nq, N, D,

@@ -53,3 +53,25 @@ def test_decode_groups_parity(case):
     err = float((o.double() - ref).norm() / ref.norm())
     print(f"[parity] decode groups {case}: rel {err:.2e}", flush=True)
     assert err <= (2.0 ** -11 if dt == "fp16" else 2.0 ** -8)
+
+
+@pytest.mark.parametrize("Nq,N,D,splits", [(40, 2144, 64, 0), (9, 1024, 128, 0), (64, 544, 64, 3)])
+def test_decode_unscaled_queries_in_parts(Nq, N, D, splits):
+    """fp16 with scale 1.0: Q as given, one wave per 32 queries, no key groups."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from grammar.attention import decode_splits, flash_attention_decode
+    assert splits or decode_splits(1, 2, Nq, N, groups=False) > 1
+    print(f"[case] decode unscaled Nq={Nq} N={N} D={D} splits={splits}", flush=True)
+    g = torch.Generator("cpu").manual_seed(43)
+    # scores of unit variance, climbing by 2 over the keys
+    q = torch.randn((1, 2, Nq, D), generator=g)
+    k = (torch.randn((1, 2, N, D), generator=g) + (torch.arange(N).float() * 2 / N).view(1, 1, -1, 1)) / D ** 0.5
+    v = torch.randn((1, 2, N, D), generator=g)
+    q, k, v = (t.half().cuda() for t in (q, k, v))
+    o = flash_attention_decode(q, k, v, scale=1.0, splits=splits)
+    torch.cuda.synchronize()
+    ref = torch.softmax(q.double() @ k.double().transpose(2, 3).contiguous(), dim=-1) @ v.double()
+    err = float((o.double() - ref).norm() / ref.norm())
+    print(f"[parity] decode unscaled: rel {err:.2e}", flush=True)
+    assert err <= 2.0 ** -11
