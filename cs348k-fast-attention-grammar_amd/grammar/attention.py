@@ -235,34 +235,55 @@ def flash_attention(q, k, v, *, causal: bool = False, scale: float | None = None
     return _FLASH_FN.apply(q, k, v, causal, scale)
 
 
-def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256, *, groups: bool = True) -> int:
+def decode_splits(B: int, H: int, Nq: int, N: int, cu_count: int = 256, *, D: int = 64, groups: bool = True) -> int:
     """Key parts per query tile for gr_attn_decode, by the kernel that runs
-    (lines measured over B H 1-64, N 256-8192, both head dims):
-    1 query (streaming kernel): one workgroup per compute unit, parts of at
-    least 256 keys; up to 512 keys one launch is faster than two (D 64 N 512:
-    5.0 us against 7.2). 2 to 4 queries (the same kernel, more arithmetic per
-    key): two workgroups per compute unit and parts of 64 keys (B H 8, N 3104:
-    12.6 us at 32 parts, 20.6 at 6), one part up to 256 keys. With heads for more
-    than half the compute units both are bound by memory and take one workgroup
-    per compute unit and parts of 512 keys (B H 180, N 832: 17.1 us in one
-    part, 19.3 in two; B H 182, N 3072, 2 queries: 59 in two, 68 in three),
-    except 2 to 4 queries below 1,024 keys and one head per unit. 5 to 64 queries
-    (flash body, four key groups per workgroup): one workgroup per compute
-    unit, at most 16 parts of at least 256 keys (B H 16, N 8192: 13.2 us at 16
-    parts, 15.9 at 32). More, and the kernel without key groups (groups=False:
-    fp16 with scale log2(e) > 1): two workgroups per compute unit, each part
-    keeping at least four 64-key tiles (without groups B H 129, N 8192, D 64: 52
-    us in four parts, 153 in one)."""
+    (lines measured over B H 1-512, N 128-16384, both head dims, every count of
+    parts; in brackets the time over the best count's, geometric mean):
+    1 query (streaming kernel): as many parts as fit one workgroup per compute
+    unit, of at least 256 keys; up to 512 keys one launch is faster than two (D
+    64 N 512: 5.0 us against 7.2) [1.02].
+    With heads for a third of the units the second launch pays from 1,024 keys
+    on (B H 128, N 768, D 64: 7.2 us in one part, 8.6 in two).
+    2 to 4 queries (the same kernel for 2 or 4, more arithmetic per key): up to
+    1.5 workgroups per compute unit for 2, 2 for 4 and with heads for more than
+    half the units. Parts pay by their work, queries x keys x D: above 2^16,
+    at least half of that a part (B H 8, N 3104, 4 queries, D 64: 12.6 us at 32
+    parts, 20.6 at 6); with heads for more than half the units from 2^18 on (B H
+    255, N 512, 4 queries, D 64: 12.3 us in one part, 17.6 in three) [1.03].
+    5 to 64 queries (flash body, four key groups per workgroup): one workgroup
+    per compute unit, at most 16 parts of at least 256 keys (B H 16, N 8192: 13.2
+    us at 16 parts, 15.9 at 32). Heads for more than half the units take one part,
+    except where two to four long ones take three quarters of its rounds of
+    resident workgroups or less (two per unit at D 64, one at D 128: B H 150, N
+    8192, D 128 137 us in one part, 121 in three; N 2048 31 and 37) [1.02].
+    More, and the kernel without key groups (groups=False: fp16 with scale
+    log2(e) > 1): two workgroups per compute unit, each part keeping at least
+    four 64-key tiles (without groups B H 129, N 8192, D 64: 52 us in four parts,
+    153 in one)."""
     heads = B * H
-    if Nq <= 4 and 2 * heads > cu_count and (Nq == 1 or N >= 1024 or heads >= cu_count):
-        return max(1, min(-(-cu_count // heads), N // 512))
+    many = 2 * heads > cu_count
     if Nq == 1:
-        return 1 if N <= 512 else max(1, min(-(-cu_count // heads), N // 256, 32))
+        if N <= 512 or (3 * heads > cu_count and N < 1024):
+            return 1
+        return max(1, min(cu_count // heads, N // 256, 32))
     if Nq <= 4:
-        return 1 if N <= 256 else max(1, min(-(-2 * cu_count // heads), N // 64, 32))
+        slots = 2 if Nq == 2 else 4
+        work = slots * N * D
+        if work <= 1 << 16 or (many and work < 1 << 18):
+            return 1
+        per_unit = 3 if slots == 2 and not many else 4          # workgroups, in halves
+        return max(1, min(per_unit * cu_count // (2 * heads), work >> 15, 32))
     if Nq <= 64 and groups:
-        return 1 if N <= 512 else max(1, min(cu_count // (B * H), N // 256, 16))
-    tiles_q = B * H * -(-Nq // 128)
+        if N <= 512:
+            return 1
+        if not many:
+            return min(cu_count // heads, N // 256, 16)
+        resident = cu_count * (2 if D == 64 else 1)
+        for s in (2, 3, 4):
+            if N * D >= s << 18 and 4 * -(-heads * s // resident) <= 3 * s * -(-heads // resident):
+                return s
+        return 1
+    tiles_q = heads * -(-Nq // 128)
     want = -(-2 * cu_count // tiles_q)
     return max(1, min(want, N // 256 if N >= 256 else 1))
 
@@ -278,7 +299,7 @@ def decode_splits_noalloc(B: int, H: int, Nq: int, N: int, D: int, cu_count: int
     scratch array (rt.DECODE_SCRATCH_BYTES), which gr_attn_decode_noalloc
     cannot grow. One part needs no scratch."""
     L = rt.lib()
-    s = decode_splits(B, H, Nq, N, cu_count, groups=groups)
+    s = decode_splits(B, H, Nq, N, cu_count, D=D, groups=groups)
     while s > 1 and int(L.gr_attn_decode_workspace(B, H, Nq, D, s)) > rt.DECODE_SCRATCH_BYTES:
         s -= 1
     return s
@@ -304,7 +325,7 @@ def _decode_args(q, k, v, scale, splits, out, workspace, stream):
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     if splits <= 0:
-        splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0), groups=_key_groups(dtype, scale))
+        splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0), D=D, groups=_key_groups(dtype, scale))
     need = int(rt.lib().gr_attn_decode_workspace(B, H, Nq, D, splits)) if splits > 1 else 0
     if need and workspace is None:
         workspace = rt.workspace(need, q.device, stream)
