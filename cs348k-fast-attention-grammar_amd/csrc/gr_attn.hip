@@ -317,9 +317,17 @@ void decode_kernel(const gr_attn_args& a, dim3 grid, hipStream_t st) {
 }
 
 // nw 1 or 2: four key groups of 32-key tiles (a part's keys over 4 or 8 waves);
-// 4: one group of 64-key tiles, or 32 when N is not a multiple of 64.
+// 4, and one_group (D = 128 in one part): one group of 64-key tiles, or 32 when
+// N is not a multiple of 64.
 template <class T, int D, bool SPLIT>
-void decode_nw(const gr_attn_args& a, int nw, bool bn64, dim3 grid, hipStream_t st) {
+void decode_nw(const gr_attn_args& a, int nw, bool one_group, bool bn64, dim3 grid, hipStream_t st) {
+  if constexpr (D == 128 && !SPLIT)
+    if (one_group) {
+      if (nw == 1 && bn64) return decode_kernel<T, D, 64, 1, false>(a, grid, st);
+      if (nw == 1) return decode_kernel<T, D, 32, 1, false>(a, grid, st);
+      if (bn64) return decode_kernel<T, D, 64, 2, false>(a, grid, st);
+      return decode_kernel<T, D, 32, 2, false>(a, grid, st);
+    }
   if (nw == 1) decode_kernel<T, D, 32, 1, SPLIT, true, 4>(a, grid, st);
   else if (nw == 2) decode_kernel<T, D, 32, 2, SPLIT, true, 4>(a, grid, st);
   else if (bn64) decode_kernel<T, D, 64, 4, SPLIT>(a, grid, st);
@@ -336,8 +344,9 @@ void decode_stream(const gr_attn_args& a, int S, hipStream_t st) {
 // Decode-shape launch: Nq queries (any count) against N keys, non-causal, K in
 // [B, H, N, D]. Up to 4 queries: the streaming kernel (gr_flash_decode.h),
 // one workgroup per head and key part. More: the flash body with 32 queries
-// per wave: up to 64 queries, four key groups per workgroup and 32-key tiles;
-// above, four waves and 64-key tiles (32 when N is not a multiple of 64).
+// per wave: up to 64 queries, four key groups per workgroup and 32-key tiles
+// (launch_decode has the exception); above, four waves and 64-key tiles (32 when
+// N is not a multiple of 64).
 // S > 1 splits the keys over S workgroups per head (or query tile) and merges
 // their partials through the workspace.
 // Message for a workspace smaller than the key split needs: the caller's
@@ -375,14 +384,19 @@ int launch_decode(gr_attn_args a, int S, void* ws, size_t ws_bytes, bool fixed_w
   const bool unscaled = gr_is_same<T, _Float16>::value && a.scale_log2 > 1.0f;
   const int nw = unscaled ? 1 : a.Nq <= 32 ? 1 : a.Nq <= 64 ? 2 : 4;
   const long long nqt = (a.Nq + 32 * nw - 1) / (32 * nw);
-  const bool bn64 = nw == 4 && a.N % 64 == 0;
+  const long long nblk = (long long)a.B * a.H * nqt;
+  if (S < 1) S = 1;
+  // D = 128 with key groups fills a CU's LDS (128 KiB): grids of more than one
+  // workgroup per CU run in rounds, which few keys do not repay (300 heads, 32
+  // queries: N 256 18.2 us, with one group 11.2; N 512 24.9 and 26.8). D = 64
+  // has two per CU and no such line.
+  const bool one_group = D == 128 && nw < 4 && !unscaled && S == 1 && a.N < 512 && nblk > gr::cu_count();
+  const bool bn64 = (nw == 4 || one_group) && a.N % 64 == 0;
   const int bn = bn64 ? 64 : 32;
   const int tiles = a.N / bn;
-  if (S < 1) S = 1;
   if (S > tiles) S = tiles;
   a.kchunk = ((tiles + S - 1) / S) * bn;
   S = (a.N + a.kchunk - 1) / a.kchunk;         // every part gets keys
-  const long long nblk = (long long)a.B * a.H * nqt;
   if (nblk > 0x7fffffffLL || S > 65535) return gr::fail(GR_E_ARG, "gr_attn_decode: grid out of range");
   if (S > 1) {
     const size_t need = gr_attn_decode_workspace(a.B, a.H, a.Nq, D, S);
@@ -397,9 +411,9 @@ int launch_decode(gr_attn_args a, int S, void* ws, size_t ws_bytes, bool fixed_w
       else decode_kernel<T, D, 32, 1, false, false>(a, grid, st);
     }
   } else if (S > 1) {
-    decode_nw<T, D, true>(a, nw, bn64, grid, st);
+    decode_nw<T, D, true>(a, nw, false, bn64, grid, st);
   } else {
-    decode_nw<T, D, false>(a, nw, bn64, grid, st);
+    decode_nw<T, D, false>(a, nw, one_group, bn64, grid, st);
   }
   int rc = gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_attn_decode launch");
   if (rc != 0 || S == 1) return rc;

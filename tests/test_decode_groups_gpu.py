@@ -23,6 +23,9 @@ CASES = [
     (1, 1, 3, 2144, 128, "fp16", 67),     # streaming kernel, the same merge
     (1, 7, 1, 1024, 64, "bf16", 3),
     (1, 2, 100, 544, 64, "fp16", 2),      # four waves, 32-key tiles, no groups
+    (1, 300, 33, 256, 128, "bf16", 1),    # more heads than compute units, D 128, few keys: one group of 64-key tiles
+    (3, 100, 5, 480, 128, "fp16", 1),     # of 32-key tiles
+    (1, 300, 9, 512, 128, "fp16", 1),     # groups again
 ]
 
 
