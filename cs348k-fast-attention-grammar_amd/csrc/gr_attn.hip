@@ -124,6 +124,12 @@ AttnShape pick_shape(int D, bool causal, bool two_wave, long long heads, int N) 
   return best;
 }
 
+// The picked shape of a call (N a multiple of 64).
+AttnShape pick_call(int dtype, int D, bool causal, bool kt, bool train, long long heads, int N) {
+  const bool w2 = dtype == GR_F16 && D == 64 && !causal, w2h = D == 128 && kt && !train;
+  return pick_shape(D, causal, N % 256 == 0 && (w2 || w2h), heads, N);
+}
+
 // Tile configurations compiled into the library: (block_m, block_n) ->
 // (waves, query blocks per wave, key tile). One wave per 32 queries.
 // block_m = block_n = 0 runs the picked shape (N a multiple of 64); where that
@@ -135,10 +141,9 @@ template <class T, int D, bool CAUSAL, bool KT>
 int dispatch_tiles(const gr_attn_args& a, int bm, int bn, hipStream_t st) {
   constexpr bool W2 = gr_is_same<T, _Float16>::value && D == 64 && !CAUSAL;
   if (bm == 0 && bn == 0 && a.N % 64 == 0) {
-    const bool two_wave = a.N % 256 == 0 && (W2 || (D == 128 && KT && a.lse == nullptr));
-    const AttnShape s = pick_shape(D, CAUSAL, two_wave, (long long)a.B * a.H, a.N);
-    if (s.kg > 1)
-      return gr::launch_flash_groups(a, gr_is_same<T, _Float16>::value ? GR_F16 : GR_BF16, D, CAUSAL, KT, s.nw, s.kg, st);
+    constexpr int DT = gr_is_same<T, _Float16>::value ? GR_F16 : GR_BF16;
+    const AttnShape s = pick_call(DT, D, CAUSAL, KT, a.lse != nullptr, (long long)a.B * a.H, a.N);
+    if (s.kg > 1) return gr::launch_flash_groups(a, DT, D, CAUSAL, KT, s.nw, s.kg, st);
     if constexpr (D == 64 && !CAUSAL)
       if (s.bn == 128) return launch_flash<T, D, 128, 4, 1, CAUSAL, KT>(a, st);
     if (s.nw == 2) return launch_flash<T, D, 64, 2, 1, CAUSAL, KT>(a, st, true);
@@ -488,6 +493,19 @@ extern "C" int gr_attn_fwd(const void* q, const void* k, const void* v, void* o,
                            int k_transposed, int causal, float scale, int block_m, int block_n, void* stream) {
   return attn_fwd(q, k, v, o, nullptr, dtype, B, H, N, D, qs, ks, vs, os, k_transposed, causal, scale, block_m,
                   block_n, stream);
+}
+
+extern "C" int gr_attn_fwd_shape(int dtype, int B, int H, int N, int D, int k_transposed, int causal, int train,
+                                 int* out3) {
+  if (!out3) return gr::fail(GR_E_ARG, "gr_attn_fwd_shape: null output");
+  if ((dtype != GR_F16 && dtype != GR_BF16) || (D != 64 && D != 128) || B <= 0 || H <= 0 || N <= 0 || N % 64)
+    return gr::fail(GR_E_ARG, "gr_attn_fwd_shape: no pick for dtype %d, D=%d, N=%d (fp16 or bf16, D 64 or 128, N a multiple of 64)",
+                    dtype, D, N);
+  const AttnShape s = pick_call(dtype, D, causal != 0, k_transposed != 0, train != 0, (long long)B * H, N);
+  out3[0] = 32 * s.nw;
+  out3[1] = s.kg;
+  out3[2] = s.bn;
+  return GR_OK;
 }
 
 extern "C" int gr_attn_fwd_train(const void* q, const void* k, const void* v, void* o, float* lse, int dtype, int B,

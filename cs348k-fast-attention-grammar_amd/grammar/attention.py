@@ -36,6 +36,17 @@ def default_tiles(N: int, D: int, dtype: str | None = None, causal: bool = False
     return bm, bn
 
 
+def picked_shape(B: int, H: int, N: int, D: int, dtype: str, *, causal: bool = False, k_transposed: bool = False,
+                 train: bool = False) -> tuple:
+    """(queries, key groups, keys per tile) of the workgroup that gr_attn_fwd (or
+    gr_attn_fwd_train) runs when no tile is named; N a multiple of 64, dtype "fp16"
+    (scale log2(e) <= 1) or "bf16". Host arithmetic."""
+    out = (ctypes.c_int * 3)()
+    rt.check(rt.lib().gr_attn_fwd_shape(rt.GR_F16 if dtype == "fp16" else rt.GR_BF16, B, H, N, D, int(k_transposed),
+                                        int(causal), int(train), out), "gr_attn_fwd_shape")
+    return tuple(out)
+
+
 def _fwd_args(q, k, v, lse, causal, scale, k_transposed, block_m, block_n, out, stream):
     """(C arguments, out) of gr_attn_fwd, or (lse given) of gr_attn_fwd_train,
     after checking the operands."""

@@ -151,6 +151,13 @@ int gr_attn_fwd(const void* q, const void* k, const void* v, void* o, int dtype,
                 const long long* v_strides, const long long* o_strides, int k_transposed,
                 int causal, float scale, int block_m, int block_n, void* stream);
 
+/* The workgroup that gr_attn_fwd (train != 0: gr_attn_fwd_train) picks for
+ * block_m = block_n = 0 at scale log2(e) <= 1: out3 = {queries, key groups, keys
+ * per tile}. GR_F16 or GR_BF16, N a multiple of 64. A 256-query pick that divides
+ * N runs the named default tile. Host arithmetic on the current device's CU count
+ * (256 without a device). No counterpart in the reference. */
+int gr_attn_fwd_shape(int dtype, int B, int H, int N, int D, int k_transposed, int causal, int train, int* out3);
+
 /* Training forward: gr_attn_fwd that also writes, per query row, the
  * log-sum-exp of the scaled (masked) scores, natural log, into lse
  * [B*H][N] fp32 (4-byte aligned) for gr_attn_bwd. No counterpart in the

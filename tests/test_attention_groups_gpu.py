@@ -36,38 +36,45 @@ def _reference(q, k, v, causal):
 
 
 CASES = [
-    # B, H, N, D, dtype, causal, k_transposed
-    (1, 1, 64, 64, "fp16", False, False),     # one query tile of 4 waves, half of them past the end
-    (1, 1, 192, 64, "bf16", True, False),     # 1 wave x 4 groups
-    (1, 3, 320, 64, "fp16", True, True),      # 10 key tiles: groups of unequal count
-    (2, 2, 512, 64, "bf16", False, True),
-    (1, 1, 2048, 64, "fp16", True, False),    # 1 wave x 8 groups
-    (1, 2, 1344, 64, "bf16", False, False),
-    (1, 15, 2432, 64, "bf16", False, False),   # 128-query tiles of 128 keys
-    (1, 16, 1024, 64, "fp16", False, False),  # 2 waves x 2 groups
-    (1, 32, 320, 64, "bf16", True, True),
-    (1, 12, 1408, 64, "bf16", False, False),  # 4 waves x 2 groups
-    (2, 32, 448, 64, "fp16", True, True),     # the last tile half-filled
-    (1, 48, 704, 64, "bf16", False, True),    # 256-query tiles, ragged
-    (2, 32, 1344, 64, "fp16", False, False),  # 128-query tiles, one group, ragged
-    (3, 16, 1344, 64, "fp16", False, True),   # 64-query tiles, one group
-    (1, 1, 64, 128, "bf16", True, False),
-    (1, 2, 320, 128, "fp16", True, True),     # 2 waves x 4 groups
-    (1, 12, 1344, 128, "bf16", False, True),
-    (1, 3, 1984, 128, "fp16", False, False),
-    (2, 32, 384, 128, "bf16", True, False),   # 4 waves x 2 groups
-    (1, 12, 1408, 128, "fp16", False, True),
-    (2, 12, 1344, 128, "bf16", False, False),  # 64-query tiles, one group
-    (2, 32, 1344, 128, "fp16", True, True),   # 256-query causal tiles, ragged
-    (1, 32, 1344, 128, "fp16", False, False),  # 256-query tiles, ragged
+    # B, H, N, D, dtype, causal, k_transposed, the picked (queries, key groups, keys per tile)
+    (1, 1, 64, 64, "fp16", False, False, (128, 1, 64)),  # one query tile of 4 waves, half of them past the end
+    (1, 1, 192, 64, "bf16", True, False, (32, 4, 32)),  # 1 wave x 4 groups
+    (1, 3, 320, 64, "fp16", True, True, (32, 4, 32)),  # 10 key tiles: groups of unequal count
+    (2, 2, 512, 64, "bf16", False, True, (32, 4, 32)),
+    (1, 1, 2048, 64, "fp16", True, False, (32, 8, 32)),  # 1 wave x 8 groups
+    (1, 2, 1344, 64, "bf16", False, False, (32, 4, 32)),
+    (1, 15, 2432, 64, "bf16", False, False, (64, 2, 64)),
+    (1, 86, 640, 64, "bf16", False, False, (128, 1, 128)),  # 128-query tiles of 128 keys
+    (1, 86, 640, 64, "fp16", False, True, (128, 1, 128)),
+    (1, 16, 1024, 64, "fp16", False, False, (64, 2, 64)),  # 2 waves x 2 groups
+    (1, 32, 320, 64, "bf16", True, True, (64, 2, 64)),
+    (1, 12, 1408, 64, "bf16", False, False, (128, 2, 64)),  # 4 waves x 2 groups
+    (2, 32, 448, 64, "fp16", True, True, (128, 2, 64)),  # the last tile half-filled
+    (1, 48, 704, 64, "bf16", False, True, (256, 1, 64)),  # 256-query tiles, ragged
+    (2, 32, 1344, 64, "fp16", False, False, (128, 1, 64)),  # 128-query tiles, one group, ragged
+    (3, 16, 1344, 64, "fp16", False, True, (64, 1, 64)),  # 64-query tiles, one group
+    (1, 1, 64, 128, "bf16", True, False, (128, 1, 64)),
+    (1, 2, 320, 128, "fp16", True, True, (64, 4, 32)),  # 2 waves x 4 groups
+    (1, 12, 1344, 128, "bf16", False, True, (64, 4, 32)),
+    (1, 3, 1984, 128, "fp16", False, False, (64, 4, 32)),
+    (2, 32, 384, 128, "bf16", True, False, (128, 2, 64)),  # 4 waves x 2 groups
+    (1, 12, 1408, 128, "fp16", False, True, (128, 2, 64)),
+    (2, 12, 1344, 128, "bf16", False, False, (64, 1, 64)),  # 64-query tiles, one group
+    (2, 32, 1344, 128, "fp16", True, True, (128, 1, 64)),
+    (1, 85, 960, 128, "fp16", True, True, (256, 1, 64)),  # 256-query causal tiles, ragged
+    (1, 85, 960, 128, "bf16", True, False, (256, 1, 64)),
+    (1, 32, 1344, 128, "fp16", False, False, (256, 1, 64)),  # 256-query tiles, ragged
 ]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c)))
 def test_picked_shape_parity(case):
     dev = _cuda()
-    from grammar.attention import flash_attention_fwd, flash_attention_fwd_train
-    B, H, N, D, dt, causal, kt = case
+    from grammar.attention import flash_attention_fwd, flash_attention_fwd_train, picked_shape
+    B, H, N, D, dt, causal, kt, shape = case
+    assert picked_shape(B, H, N, D, dt, causal=causal, k_transposed=kt) == shape
+    if not kt:
+        assert picked_shape(B, H, N, D, dt, causal=causal, train=True) == shape
     print(f"[case] picked attention {case}", flush=True)
     g = torch.Generator("cpu").manual_seed(19)
     q, k, v = (torch.randn((B, N, H, D), generator=g).to(DT[dt]).to(dev).transpose(1, 2) for _ in range(3))
@@ -87,6 +94,21 @@ def test_picked_shape_parity(case):
         torch.cuda.synchronize()
         assert float((o2.double() - ref).norm() / ref.norm()) <= U[dt]
         assert float((lse.double() - lse_ref).abs().max()) <= 2e-3
+
+
+def test_part_filled_256_query_causal_tiles_at_head_dim_64():
+    dev = _cuda()
+    from grammar.attention import flash_attention_fwd_train, picked_shape
+    H, N, D = 122, 4032, 64
+    assert picked_shape(1, H, N, D, "bf16", causal=True, train=True) == (256, 1, 64)
+    print(f"[case] picked attention {H} heads N {N} D {D} causal", flush=True)
+    g = torch.Generator("cuda").manual_seed(29)
+    q, k, v = (torch.randn((1, H, N, D), generator=g, device=dev).bfloat16() for _ in range(3))
+    o, lse = flash_attention_fwd_train(q, k, v, causal=True)
+    for h in (0, 61, H - 1):
+        ref, lse_ref = _reference(q[:, h:h + 1], k[:, h:h + 1], v[:, h:h + 1], True)
+        assert float((o[:, h:h + 1].double() - ref).norm() / ref.norm()) <= U["bf16"]
+        assert float((lse[:, h:h + 1].double() - lse_ref).abs().max()) <= 2e-3
 
 
 @pytest.mark.parametrize("D,N,causal,dt", [(64, 448, False, "fp16"), (64, 2048, True, "fp16"), (128, 832, False, "bf16"),
