@@ -62,9 +62,9 @@ int launch_w2h(const gr_attn_args& a, hipStream_t st) {
 // us per iteration that a CU sustains and `lat` the us that one workgroup
 // alone takes. The constants are fitted to 2,300 launches (B H 1-64, N 64-4096,
 // both head dims, fp16 and bf16, causal or not); the pick is within 0.9 % of
-// the fastest shape (geometric mean, 19 % at worst) and takes 0.77x the time
-// of the largest tile that divides N, which ran before. The 256-query tile
-// that divides N is preferred within the model's error (5 %).
+// the fastest shape (geometric mean, 19 % at worst of those) and takes 0.77x
+// the time of the largest tile that divides N, which ran before. The 256-query
+// tile that divides N is preferred within the model's error (5 %).
 struct AttnShape {
   int nw, kg, bn;
   double lat, thr, t0, t1;
@@ -108,6 +108,14 @@ AttnShape pick_shape(int D, bool causal, bool two_wave, long long heads, int N) 
     const double alone = iters * s.lat, shared = rounds * mean * s.thr;
     double t = s.t0 + (alone > shared ? alone : shared) + s.t1 * rounds;
     if (s.nw == 8 && N % 256 == 0) t *= 0.95;
+    // Many short workgroups of 64 x 64: up to five are resident on a CU and
+    // hide each other's start and end, which t0 and t1 count in full, while a
+    // larger tile that does not divide N is part empty (200 heads, N 320, bf16:
+    // 10.1 us, 13.1 on 128 x 64; 300 heads, N 192, causal 8.4 and 10.8).
+    if (D == 64 && s.nw == 2 && s.kg == 1 && w > 3. * cus && iters <= 7 && N % 128 == 64) t *= 0.8;
+    // 64 queries x 2 groups take 64 KiB of LDS, so from two workgroups per CU on
+    // the rest wait (12 heads, N 4096, bf16: 75 us, 66 on 256 x 128)
+    if (!causal && D == 64 && s.nw == 2 && s.kg == 2 && w > 2. * cus) t *= 1.1;
     if (t < best_t) {
       best_t = t;
       best = s;

@@ -43,7 +43,7 @@ CASES = [
     (2, 2, 512, 64, "bf16", False, True, (32, 4, 32)),
     (1, 1, 2048, 64, "fp16", True, False, (32, 8, 32)),  # 1 wave x 8 groups
     (1, 2, 1344, 64, "bf16", False, False, (32, 4, 32)),
-    (1, 15, 2432, 64, "bf16", False, False, (64, 2, 64)),
+    (1, 15, 2432, 64, "bf16", False, False, (128, 1, 128)),
     (1, 86, 640, 64, "bf16", False, False, (128, 1, 128)),  # 128-query tiles of 128 keys
     (1, 86, 640, 64, "fp16", False, True, (128, 1, 128)),
     (1, 16, 1024, 64, "fp16", False, False, (64, 2, 64)),  # 2 waves x 2 groups
