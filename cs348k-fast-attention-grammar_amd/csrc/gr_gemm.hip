@@ -111,6 +111,10 @@ gr::GemmPlan pick_plan(int batch, int M, int N, int K, size_t ws_max) {
   gr::GemmPlan best = {256, 256, 1, 0};
   const int cus = gr::cu_count();
   if (cus <= 0) return best;
+  // Few k tiles and a C of more than half a round of 256 x 256 tiles: bound by
+  // its store, which the model does not count (K 64: M 1024, N 11008 10.7 us,
+  // 13.1 on 256 x 128; M 4096, N 4096 12.0 and 14.0 on 128 x 128)
+  if (K < 256 && 2LL * batch * ((M + 255) / 256) * ((N + 255) / 256) > cus) return best;
   double best_t = 1e30;
   for (const TileModel& m : K % 64 == 0 ? kTiles64 : kTiles32) {
     // The 32-row tile reads B once per 32 rows: up to 32, or 64 while a short K

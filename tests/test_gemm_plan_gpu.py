@@ -38,6 +38,8 @@ CASES = [
     (1, 200, 4104, 8224, "bf16", "none", True, True),     # and on 32-deep k tiles
     (1, 1000, 520, 64, "fp16", "relu", False, False),     # 256 x 128
     (1, 520, 3000, 96, "bf16", "none", False, False),     # 128 x 128, 32-deep k tiles
+    (1, 700, 11000, 64, "bf16", "silu", False, False),    # bound by the store of C: 256 x 256
+    (2, 1000, 8200, 224, "fp16", "none", True, False),    # 32-deep k tiles
 ]
 
 
