@@ -223,18 +223,12 @@ int launch_gemm_f32_groups(const gr_gemm_args& a, int batch, hipStream_t st) {
   return gr::hip_check(hipGetLastError(), GR_E_LAUNCH, "gr_gemm launch");
 }
 
-// Whether the k-group body takes a call whose tile is bm x bn: matrix-core
-// cycles per SIMD of the launch's rounds (64 per 32x32x2 MFMA) less than 0.8
-// of the tile's. _gemm_f32_groups in the renderer is the same rule.
+// Whether the k-group body takes a call whose tile is bm x bn (gr_gemm_f32_groups
+// is the rule).
 bool f32_groups(const gr_gemm_args& a, int batch, int bm, int bn) {
+  if (a.M % 32 || a.N % 32) return false;
   const int cus = gr::cu_count();
-  if (cus <= 0 || a.M % 32 || a.N % 32) return false;
-  const int waves = (bm >= 64 ? 2 : 1) * (bn >= 64 ? 2 : 1);
-  const long long tiles = (long long)batch * ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn);
-  const long long blocks = (long long)batch * (a.M / 32) * (a.N / 32);
-  const long long chain = (long long)(bm / 32) * (bn / 32) / waves;       // 32 x 32 blocks per wave
-  const int nk = a.K / (a.K % 16 == 0 ? 16 : 8);                          // k tiles, (nk + 3) / 4 per group
-  return 10 * ((blocks + cus - 1) / cus) * ((nk + 3) / 4) < 8 * ((tiles + cus - 1) / cus) * chain * nk;
+  return cus > 0 && gr_gemm_f32_groups(batch, a.M, a.N, a.K / (a.K % 16 == 0 ? 16 : 8), bm, bn, cus) == 1;
 }
 
 template <bool KM, int EPI>
@@ -325,6 +319,21 @@ int mlp_fwd(const void* x, const void* w1, const void* w2, void* h, void* y, int
 }
 
 }  // namespace
+
+// Matrix-core time per SIMD of the launch's rounds, in 32 x 32 blocks x k tiles,
+// with one more a round for its start and merge: below 0.7 of the tile's. Of
+// 1,324 shapes (M, N 32-4096, K 32-4096) the chosen ones take 0.35x the tile's
+// time (geometric mean) and none over 1.04x; a line at 0.8 without the round's
+// one had 17 of them at 1.05-1.45x (M 768, N 4096, K 1024: 79 us on 192 tiles of
+// 128 x 128, 98 on 3,072 blocks).
+extern "C" int gr_gemm_f32_groups(int batch, int M, int N, int ktiles, int block_m, int block_n, int cus) {
+  if (batch <= 0 || M <= 0 || N <= 0 || ktiles <= 0 || block_m < 32 || block_n < 32 || cus <= 0) return 0;
+  const int waves = (block_m >= 64 ? 2 : 1) * (block_n >= 64 ? 2 : 1);
+  const long long tiles = (long long)batch * ((M + block_m - 1) / block_m) * ((N + block_n - 1) / block_n);
+  const long long blocks = (long long)batch * (M / 32) * (N / 32);
+  const long long chain = (long long)(block_m / 32) * (block_n / 32) / waves;       // 32 x 32 blocks per wave
+  return 10 * ((blocks + cus - 1) / cus) * ((ktiles + 3) / 4 + 1) < 7 * ((tiles + cus - 1) / cus) * (chain * ktiles + 1);
+}
 
 extern "C" int gr_gemm(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K,
                        const long long* a_strides, const long long* b_strides, const long long* c_strides,

@@ -532,14 +532,14 @@ GEMM_F32_GROUPS_LDS = 4 * 32 * 32 * 4      # LDS bytes of gr_gemm_f32_groups_bod
 def _gemm_f32_groups(M, N, nk, batch, bm, bn, cus=GEMM_CUS):
     """Whether an fp32 GEMM stage runs as 32 x 32 blocks with K over the four
     waves of a workgroup (gr_gemm_f32_groups_body) instead of the program's
-    tile: the library's f32_groups rule, matrix-core cycles per SIMD of the
-    launch's rounds below 0.8 of the tile's (nk k tiles over four groups).
-    64 x 64 tiles with K = 1024: 256 x 512 (32 of them) 25.1 -> 7.1 us, 512 x
-    1024 (128) 25.6 -> 17, 1024 x 1024 (256) 26 -> 33."""
+    tile: the library's rule (gr_gemm_f32_groups), matrix-core time per SIMD of
+    the launch's rounds, one k tile more a round, below 0.7 of the tile's (nk k
+    tiles over four groups). 64 x 64 tiles with K = 1024: 256 x 512 (32 of them)
+    25.1 -> 7.1 us, 512 x 1024 (128) 25.6 -> 17, 1024 x 1024 (256) 26 -> 33."""
     waves = (2 if bm >= 64 else 1) * (2 if bn >= 64 else 1)
     chain = (bm // 32) * (bn // 32) // waves            # 32 x 32 blocks per wave, nk k tiles each
-    tiles = batch * _cdiv(M, bm) * _cdiv(N, bn)
-    return 10 * _cdiv(batch * (M // 32) * (N // 32), cus) * _cdiv(nk, 4) < 8 * _cdiv(tiles, cus) * chain * nk
+    tiles, blocks = batch * _cdiv(M, bm) * _cdiv(N, bn), batch * (M // 32) * (N // 32)
+    return 10 * _cdiv(blocks, cus) * (_cdiv(nk, 4) + 1) < 7 * _cdiv(tiles, cus) * (chain * nk + 1)
 
 
 def _gemm_waves(bm, bn):

@@ -107,6 +107,7 @@ def lib() -> ctypes.CDLL:
         L.gr_gemm_workspace.restype = sz
         L.gr_gemm_ws.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, _ll2, _ll2, _ll2, i32, i32,
                                  ctypes.c_float, vp, sz, vp]
+        L.gr_gemm_f32_groups.argtypes = [i32, i32, i32, i32, i32, i32, i32]
         L.gr_mlp_fwd.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]
         L.gr_mlp_fwd_workspace.argtypes = [i32, i32, i32, i32]
         L.gr_mlp_fwd_workspace.restype = sz
@@ -136,7 +137,7 @@ EXPORTED = (
     "gr_selftest_mfma32", "gr_gemm", "gr_mlp_fwd", "gr_attn_decode_workspace", "gr_attn_decode",
     "gr_attn_fwd_train", "gr_attn_bwd_workspace", "gr_attn_bwd", "gr_attn_decode_noalloc",
     "gr_plan_run_args", "gr_gemm_workspace", "gr_gemm_ws", "gr_mlp_fwd_workspace", "gr_mlp_fwd_ws",
-    "gr_selftest_f32_no_workspace", "gr_attn_fwd_shape",
+    "gr_selftest_f32_no_workspace", "gr_attn_fwd_shape", "gr_gemm_f32_groups",
 )
 
 # Bytes of the per-device scratch array behind gr_attn_decode_noalloc (GR_DECODE_SCRATCH_BYTES).

@@ -16,3 +16,31 @@ pytest.importorskip("torch")
 def test_attention_64_query_tiles(H, N, D, causal, shape):
     from grammar.attention import picked_shape
     assert picked_shape(1, H, N, D, "bf16", causal=causal) == shape
+
+
+def test_rendered_fp32_stages_follow_the_library_rule():
+    """The rule for 32 x 32 blocks with K over four waves is written in the
+    library and in the renderer."""
+    import itertools
+    from grammar import runtime as rt
+    from grammar.hip_backend import _gemm_f32_groups
+    L = rt.lib()
+    picked = 0
+    for M, N, nk, batch, bm, bn, cus in itertools.product((32, 128, 256, 768, 4096), (64, 512, 800, 4096), (1, 4, 5, 32, 256),
+                                                          (1, 3), (32, 64, 128), (32, 64, 128), (256, 64)):
+        if M % bm == 0 and N % bn == 0:
+            want = bool(L.gr_gemm_f32_groups(batch, M, N, nk, bm, bn, cus))
+            assert _gemm_f32_groups(M, N, nk, batch, bm, bn, cus) == want, (M, N, nk, batch, bm, bn, cus)
+            picked += want
+    assert picked > 100
+
+
+@pytest.mark.parametrize("M,N,nk,bm,bn,groups", [
+    (256, 512, 64, 64, 64, True), (512, 1024, 64, 64, 64, True), (1024, 1024, 64, 64, 64, False),
+    (768, 4096, 64, 128, 128, False),      # 12 rounds of blocks against one of tiles: 98 us, 79 on the tile
+    (2048, 1024, 4, 128, 128, False),      # one k tile a wave: 11.6 us, 9.8 on the tile
+    (2048, 1024, 16, 128, 128, True),
+])
+def test_fp32_groups_lines(M, N, nk, bm, bn, groups):
+    from grammar import runtime as rt
+    assert bool(rt.lib().gr_gemm_f32_groups(1, M, N, nk, bm, bn, 256)) == groups
