@@ -305,7 +305,10 @@ def schedule_knobs(loop: ParallelLoop, program: Program) -> dict:
     query blocks per wave and pipelined schedule, the fp32 GEMM's split K,
     the 16-bit 256 x 256 GEMM's waves, the flash body with two waves per SIMD
     (which, when on, is the only flash knob offered: the other two do not
-    apply to it); empty for other stages."""
+    apply to it); empty for other stages. Two knobs are honoured without being
+    offered, as pins: "lowering": "generic", and an fp32 GEMM's "kgroups" (1: the
+    program's tile, 4: 32 x 32 blocks with K over four waves; _gemm_f32_groups
+    decides without it)."""
     f = _match_flash(loop, program)
     if f is None:
         gm = _match_gemm(loop, program)
@@ -527,6 +530,7 @@ def _gemm_f32_lds(bm, bn, bk, kmajor):
 
 
 GEMM_F32_GROUPS_LDS = 4 * 32 * 32 * 4      # LDS bytes of gr_gemm_f32_groups_body
+GEMM_KGROUPS = (1, 4)                      # values of the knob "kgroups"
 
 
 def _gemm_f32_groups(M, N, nk, batch, bm, bn, cus=GEMM_CUS):
@@ -659,11 +663,16 @@ def _match_gemm(loop: ParallelLoop, program: Program):
         ks = int((getattr(loop, "knobs", None) or {}).get("ksplit", 1))
         if ks not in GEMM_KSPLIT or K % (ks * BK) or ks * batch * M * N * 4 > GEMM_WS_LIMIT:
             ks = 1
+        # 32 x 32 blocks with K over four waves: by the shape, or pinned (knob
+        # "kgroups": 1 = the program's tile, 4 = the blocks)
+        kg = int((getattr(loop, "knobs", None) or {}).get("kgroups", 0))
+        if kg not in GEMM_KGROUPS:
+            kg = 4 if _gemm_f32_groups(M, N, K // min(BK, 16), batch, BM, BN) else 1
         return {"a": aload.source, "b": bload.source, "c": loop.out, "M": M, "N": N, "K": K, "batch": batch,
                 "a_sb": M * K if a_batched else 0, "b_sb": K * N if b_batched else 0, "c_sb": M * N,
                 "kmajor": kmajor, "act": act, "alpha": alpha, "BM": BM, "BN": BN, "BK": BK,
                 "WGM": 2 if BM >= 64 else 1, "WGN": 2 if BN >= 64 else 1, "f32": True,
-                "res": res.source if res is not None else None, "ksplit": ks}
+                "res": res.source if res is not None else None, "ksplit": ks, "kgroups": kg}
     if BM not in GEMM_WAVES_M or BN not in GEMM_WAVES_N:   # ragged M, N: edge tiles store their valid part
         return None
     BK = rl.tile if rl is not None else 64
@@ -769,7 +778,7 @@ def _render_gemm(loop, program, f) -> tuple:
         return _render_gemm_f32_split(loop, program, f, args, params, km)
     if f.get("f32"):
         nt = f["WGM"] * f["WGN"] * 64
-        groups = _gemm_f32_groups(f["M"], f["N"], f["K"] // min(f["BK"], 16), f["batch"], f["BM"], f["BN"])
+        groups = f["kgroups"] == 4
         how, kg_line = "", ""
         if groups:
             nt = 256
