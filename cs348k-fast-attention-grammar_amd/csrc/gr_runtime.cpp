@@ -11,6 +11,8 @@
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -179,17 +181,20 @@ int gr_plan_run(gr_plan* p, void* stream) {
 
 int gr_plan_run_args(gr_plan* p, void* stream, const uint64_t* args, int nargs) {
   if (!p || nargs < 0 || (nargs && !args)) return gr::fail(GR_E_ARG, "gr_plan_run_args: bad argument");
-  constexpr size_t kMax = 64;                 // arguments of one step
-  size_t total = 0;
+  size_t total = 0, most = 0;
   for (size_t i = 0; i < p->steps.size(); ++i) {
     const gr_plan_step& s = p->steps[i];
     if (!s.k) return gr::fail(GR_E_ARG, "gr_plan_run_args: step %zu not set", i);
-    if (s.args.size() > kMax) return gr::fail(GR_E_ARG, "gr_plan_run_args: step %zu has over %zu arguments", i, kMax);
     total += s.args.size();
+    if (s.args.size() > most) most = s.args.size();
   }
   if (total != (size_t)nargs) return gr::fail(GR_E_ARG, "gr_plan_run_args: %zu arguments needed, %d given", total, nargs);
+  constexpr size_t kFew = 64;                  // arguments of a step kept on the stack
+  void* few[kFew];
+  std::unique_ptr<void*[]> many(most > kFew ? new (std::nothrow) void*[most] : nullptr);
+  if (most > kFew && !many) return gr::fail(GR_E_RUNTIME, "gr_plan_run_args: no memory for %zu arguments", most);
+  void** const argp = most > kFew ? many.get() : few;
   for (const gr_plan_step& s : p->steps) {
-    void* argp[kMax];
     for (size_t a = 0; a < s.args.size(); ++a) argp[a] = const_cast<uint64_t*>(args++);
     const int rc = launch_raw(s.k, s.grid, s.block, s.lds, (hipStream_t)stream, s.args.empty() ? nullptr : argp);
     if (rc) return rc;

@@ -88,8 +88,8 @@ int gr_plan_set_step(gr_plan* p, int i, gr_kernel* k, const uint32_t grid[3], co
                      uint32_t lds_bytes, const uint64_t* args, int nargs);
 int gr_plan_run(gr_plan* p, void* stream);
 /* gr_plan_run with the arguments of this call, the steps' one after another
- * (nargs = the sum of their counts, at most 64 a step), instead of the bound
- * ones. The plan is only read: threads may run one plan at the same time. */
+ * (nargs = the sum of their counts), instead of the bound ones. The plan is
+ * only read: threads may run one plan at the same time. */
 int gr_plan_run_args(gr_plan* p, void* stream, const uint64_t* args, int nargs);
 void gr_plan_free(gr_plan* p);
 
