@@ -337,6 +337,9 @@ def _decode_args(q, k, v, scale, splits, out, workspace, stream):
         scale = 1.0 / math.sqrt(D)
     if splits <= 0:
         splits = decode_splits(B, H, Nq, N, rt.cu_count(q.device.index or 0), D=D, groups=_key_groups(dtype, scale))
+        if workspace is not None and splits > 1:      # sized by the caller: the most parts that fit, from two on
+            fit = workspace.numel() * workspace.element_size() // (int(rt.lib().gr_attn_decode_workspace(B, H, Nq, D, 2)) // 2)
+            splits = fit if 2 <= fit < splits else splits
     need = int(rt.lib().gr_attn_decode_workspace(B, H, Nq, D, splits)) if splits > 1 else 0
     if need and workspace is None:
         workspace = rt.workspace(need, q.device, stream)
@@ -406,8 +409,9 @@ def flash_attention_decode(q, k, v, *, scale: float | None = None, splits: int =
                            workspace=None, stream=None):
     """O = softmax(scale * Q K^T) V for Nq queries against N keys (non-causal):
     q [B, H, Nq, D], k and v [B, H, N, D] (N a multiple of 32), fp16/bf16 on
-    the GPU. splits = 0 picks the key split (decode_splits); the workspace
-    it needs is allocated here unless given."""
+    the GPU. splits = 0 picks the key split (decode_splits; with a workspace
+    given, at most the parts it holds); the workspace it needs is allocated
+    here unless given."""
     args, out, workspace = _decode_args(q, k, v, scale, splits, out, workspace, stream)
     rt.check(rt.lib().gr_attn_decode(*args), "gr_attn_decode")
     return out

@@ -78,3 +78,25 @@ def test_decode_unscaled_queries_in_parts(Nq, N, D, splits):
     err = float((o.double() - ref).norm() / ref.norm())
     print(f"[parity] decode unscaled: rel {err:.2e}", flush=True)
     assert err <= 2.0 ** -11
+
+
+@pytest.mark.parametrize("Nq", [1, 3, 40])
+def test_decode_default_parts_fit_a_given_workspace(Nq):
+    """splits = 0 with a workspace of fewer parts than the default takes those;
+    one that does not hold two is refused."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from grammar import runtime as rt
+    from grammar.attention import decode_splits, flash_attention_decode
+    print(f"[case] decode given workspace Nq={Nq}", flush=True)
+    H, N, D = 4, 8192, 64
+    g = torch.Generator("cpu").manual_seed(59)
+    q, kv = (torch.randn((1, H, n, D), generator=g).bfloat16().cuda() for n in (Nq, N))
+    assert decode_splits(1, H, Nq, N) > 4
+    need = int(rt.lib().gr_attn_decode_workspace(1, H, Nq, D, 4))
+    ws = torch.empty(need + 16, dtype=torch.uint8, device="cuda")
+    assert torch.equal(flash_attention_decode(q, kv, kv, workspace=ws), flash_attention_decode(q, kv, kv, splits=4))
+    big = torch.empty(64 * need, dtype=torch.uint8, device="cuda")
+    assert torch.equal(flash_attention_decode(q, kv, kv, workspace=big), flash_attention_decode(q, kv, kv))
+    with pytest.raises(ValueError):
+        flash_attention_decode(q, kv, kv, workspace=ws[:need // 4 + 16])
