@@ -45,8 +45,10 @@ constexpr long long kF32SplitTarget = 256;
 // order, so they can share it. hipStreamPerThread names a different stream in
 // every host thread, so its buffers are kept per thread as well. A split
 // launch has at most kF32SplitTarget workgroups of 32 query rows (query
-// blocks x parts), so one size holds every call's.
-constexpr size_t kF32WorkspaceBytes = (size_t)kF32SplitTarget * 32 * (128 + 2) * sizeof(float);   // 4.3 MB
+// blocks x parts), so one size holds every call's. It has two halves: the splits
+// that captured calls may take (capture_parts) have the first to themselves, so
+// that a graph replayed on another stream shares it with such calls only.
+constexpr size_t kF32WorkspaceBytes = (size_t)kF32SplitTarget * 32 * (128 + 2) * sizeof(float);   // 4.3 MB a half
 
 struct F32Workspace {
   int dev;
@@ -66,7 +68,7 @@ int f32_workspace(hipStream_t st, void** out) {
   int rc = gr::hip_check(hipGetDevice(&dev), GR_E_RUNTIME, "gr_attn_fwd: hipGetDevice");
   if (rc) return rc;
   const std::thread::id thread = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
-  size_t bytes = kF32WorkspaceBytes;
+  size_t bytes = 2 * kF32WorkspaceBytes;
   if (t_fail_workspaces > 0) {
     --t_fail_workspaces;
     bytes = (size_t)1 << 60;              // more than any device has
@@ -115,7 +117,7 @@ int launch_parts(const gr_attn_args& a, long long nblk, float* ws_o, float* ws_m
 }
 
 template <int D, bool KT, int PARTS>
-int launch_split(const gr_attn_args& a, long long nblk, hipStream_t st) {
+int launch_split(const gr_attn_args& a, long long nblk, int fixed, hipStream_t st) {
   const long long rows = (long long)a.B * a.H * a.N;
   const size_t o_floats = (size_t)PARTS * rows * D;
   std::lock_guard<std::mutex> hold(g_f32_ws_lock);
@@ -123,7 +125,7 @@ int launch_split(const gr_attn_args& a, long long nblk, hipStream_t st) {
   int rc = f32_workspace(st, &ws);
   if (rc && !capturing(st)) return launch_parts<D, KT, 1>(a, nblk, nullptr, nullptr, st);   // no memory for it
   if (rc) return rc;
-  float* ws_o = static_cast<float*>(ws);
+  float* ws_o = static_cast<float*>(ws) + (PARTS == fixed ? 0 : kF32WorkspaceBytes / sizeof(float));
   float* ws_ml = ws_o + o_floats;
   rc = launch_parts<D, KT, PARTS>(a, nblk, ws_o, ws_ml, st);
   if (rc) return rc;
@@ -177,9 +179,9 @@ int launch_flash32(const gr_attn_args& a, hipStream_t st) {
   int parts = pick_parts(D, nblk, a.N / 32);
   const int fixed = capture_parts(nblk, a.N);
   if (parts > 1 && parts != fixed && capturing(st)) parts = fixed;
-  if (parts == 8) return launch_split<D, KT, 8>(a, nblk, st);
-  if (parts == 4) return launch_split<D, KT, 4>(a, nblk, st);
-  if (parts == 2) return launch_split<D, KT, 2>(a, nblk, st);
+  if (parts == 8) return launch_split<D, KT, 8>(a, nblk, fixed, st);
+  if (parts == 4) return launch_split<D, KT, 4>(a, nblk, fixed, st);
+  if (parts == 2) return launch_split<D, KT, 2>(a, nblk, fixed, st);
   return launch_parts<D, KT, 1>(a, nblk, nullptr, nullptr, st);
 }
 

@@ -122,12 +122,13 @@ int gr_plan_time(gr_plan* p, void* stream, int warmup, int iters, int mode, floa
  *  2, 4 or 8 workgroups (the library picks by D, N, the query blocks and the
  *  CU count) and a second launch merges their partials, which sit in a
  *  workspace the library allocates once per (device, stream) and keeps until
- *  the process ends: 4.3 MB, for a split launch has at most 256 workgroups of
- *  32 queries. On the per-thread default stream each host thread has its own.
- *  Without memory for it the call runs unsplit. Under capture only N a
- *  multiple of 256 with at most 128 query blocks is split, over the most of 8,
- *  4 or 2 workgroups that divide N / 128; call once on a stream before
- *  capturing such calls into a graph.
+ *  the process ends: 8.5 MB, for a split launch has at most 256 workgroups of
+ *  32 queries (4.3 MB), and the splits below have memory of their own. On the
+ *  per-thread default stream each host thread has its own. Without memory for
+ *  it the call runs unsplit. Under capture only N a multiple of 256 with at
+ *  most 128 query blocks is split, over the most of 8, 4 or 2 workgroups that
+ *  divide N / 128; call once on a stream before capturing such calls into a
+ *  graph, and order its replays on other streams with calls of such splits.
  *  Q, V, O: [B, H, N, D] with strides {batch, head, seq} in elements
  *  (unit stride along D). K: [B, H, N, D] if k_transposed == 0, else KT
  *  [B, H, D, N] whose k_strides = {batch, head, d} (unit stride along N).

@@ -120,3 +120,37 @@ def test_fp32_split_without_memory_for_its_workspace(heads, N, D):
     torch.cuda.synchronize()
     _check(whole, q, k, v, ("no workspace", heads, N, D))
     assert torch.equal(split, again)
+
+
+def test_fp32_graph_replay_beside_eager_splits():
+    """A captured split's partials are not those of eager calls that split in
+    other shapes on the capturing stream: replayed on another stream beside them,
+    both keep their results."""
+    dev = _cuda()
+    from grammar.attention import bind_flash_attention
+    graph_in, eager_in = _inputs(1, 512, 64, dev), _inputs(4, 320, 64, dev, seed=42)
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    print("[case] fp32 graph replay beside eager splits", flush=True)
+    with torch.cuda.stream(s):
+        s.wait_stream(torch.cuda.default_stream())
+        run, out = bind_flash_attention(*graph_in, stream=s)
+        eager, eout = bind_flash_attention(*eager_in, stream=s)
+        run()
+        eager()
+        s.synchronize()
+        want, ewant = out.clone(), eout.clone()
+        s.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            run()
+    for _ in range(20):
+        out.zero_()
+        eout.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(t):
+            for _ in range(8):
+                graph.replay()
+        for _ in range(8):
+            eager()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(eout, ewant)
