@@ -225,10 +225,10 @@ int launch_gemm_f32_groups(const gr_gemm_args& a, int batch, hipStream_t st) {
 
 // Whether the k-group body takes a call whose tile is bm x bn (gr_gemm_f32_groups
 // is the rule).
-bool f32_groups(const gr_gemm_args& a, int batch, int bm, int bn) {
+bool f32_groups(const gr_gemm_args& a, int batch, bool km, int bm, int bn) {
   if (a.M % 32 || a.N % 32) return false;
   const int cus = gr::cu_count();
-  return cus > 0 && gr_gemm_f32_groups(batch, a.M, a.N, a.K / (a.K % 16 == 0 ? 16 : 8), bm, bn, cus) == 1;
+  return cus > 0 && gr_gemm_f32_groups(batch, a.M, a.N, a.K / (a.K % 16 == 0 ? 16 : 8), km, bm, bn, cus) == 1;
 }
 
 template <bool KM, int EPI>
@@ -236,7 +236,7 @@ int dispatch_f32_tile(const gr_gemm_args& a, int batch, int bm, int bn, hipStrea
   const bool pick = bm == 0 && bn == 0;
   if (bm == 0) bm = a.M % 128 == 0 ? 128 : a.M % 64 == 0 ? 64 : 32;
   if (bn == 0) bn = a.N % 128 == 0 ? 128 : a.N % 64 == 0 ? 64 : 32;
-  if (pick && f32_groups(a, batch, bm, bn)) return launch_gemm_f32_groups<KM, EPI>(a, batch, st);
+  if (pick && f32_groups(a, batch, KM, bm, bn)) return launch_gemm_f32_groups<KM, EPI>(a, batch, st);
 #define GR_T(M_, N_) \
   if (bm == M_ && bn == N_) return launch_gemm_f32<M_, N_, KM, EPI>(a, batch, st);
   GR_T(32, 32) GR_T(32, 64) GR_T(32, 128) GR_T(64, 32) GR_T(64, 64) GR_T(64, 128)
@@ -320,19 +320,24 @@ int mlp_fwd(const void* x, const void* w1, const void* w2, void* h, void* y, int
 
 }  // namespace
 
-// Matrix-core time per SIMD of the launch's rounds, in 32 x 32 blocks x k tiles,
-// with one more a round for its start and merge: below 0.7 of the tile's. Of
-// 1,324 shapes (M, N 32-4096, K 32-4096) the chosen ones take 0.35x the tile's
-// time (geometric mean) and none over 1.04x; a line at 0.8 without the round's
-// one had 17 of them at 1.05-1.45x (M 768, N 4096, K 1024: 79 us on 192 tiles of
-// 128 x 128, 98 on 3,072 blocks).
-extern "C" int gr_gemm_f32_groups(int batch, int M, int N, int ktiles, int block_m, int block_n, int cus) {
+// Two lines. Matrix-core time per SIMD of the launch's rounds, in 32 x 32 blocks x
+// k tiles, below 0.8 of the tile's; and few rounds, since blocks read their
+// operands without sharing them: up to two per 32 x 32 block that a wave of the
+// tile owns (a third where it owns one and B is not K-major), four where the tile
+// has two waves, which leave half of a CU's SIMDs idle. Over 11,054 pairs of shape
+// and tile (M, N 64-4096, K 32-2048; tiles of 32, 64, 128 a side) the choice is
+// within 0.6 % of the faster body (geometric mean; 2.3 % with the first line
+// alone, which took M 768, N 4096, K 1024 from 79 us on 128 x 128 to 98 and
+// 4096 x 512, K 64 K-major on 32 x 32 from 7.0 to 11.8).
+extern "C" int gr_gemm_f32_groups(int batch, int M, int N, int ktiles, int b_kmajor, int block_m, int block_n, int cus) {
   if (batch <= 0 || M <= 0 || N <= 0 || ktiles <= 0 || block_m < 32 || block_n < 32 || cus <= 0) return 0;
   const int waves = (block_m >= 64 ? 2 : 1) * (block_n >= 64 ? 2 : 1);
   const long long tiles = (long long)batch * ((M + block_m - 1) / block_m) * ((N + block_n - 1) / block_n);
   const long long blocks = (long long)batch * (M / 32) * (N / 32);
   const long long chain = (long long)(block_m / 32) * (block_n / 32) / waves;       // 32 x 32 blocks per wave
-  return 10 * ((blocks + cus - 1) / cus) * ((ktiles + 3) / 4 + 1) < 7 * ((tiles + cus - 1) / cus) * (chain * ktiles + 1);
+  const long long rounds = (blocks + cus - 1) / cus;
+  if (rounds > (waves == 2 ? 4 * chain : 2 * chain + (chain == 1 && !b_kmajor))) return 0;
+  return 10 * rounds * ((ktiles + 3) / 4) < 8 * ((tiles + cus - 1) / cus) * chain * ktiles;
 }
 
 extern "C" int gr_gemm(const void* a, const void* b, void* c, int dtype, int batch, int M, int N, int K,

@@ -533,17 +533,20 @@ GEMM_F32_GROUPS_LDS = 4 * 32 * 32 * 4      # LDS bytes of gr_gemm_f32_groups_bod
 GEMM_KGROUPS = (1, 4)                      # values of the knob "kgroups"
 
 
-def _gemm_f32_groups(M, N, nk, batch, bm, bn, cus=GEMM_CUS):
+def _gemm_f32_groups(M, N, nk, batch, kmajor, bm, bn, cus=GEMM_CUS):
     """Whether an fp32 GEMM stage runs as 32 x 32 blocks with K over the four
     waves of a workgroup (gr_gemm_f32_groups_body) instead of the program's
-    tile: the library's rule (gr_gemm_f32_groups), matrix-core time per SIMD of
-    the launch's rounds, one k tile more a round, below 0.7 of the tile's (nk k
-    tiles over four groups). 64 x 64 tiles with K = 1024: 256 x 512 (32 of them)
-    25.1 -> 7.1 us, 512 x 1024 (128) 25.6 -> 17, 1024 x 1024 (256) 26 -> 33."""
+    tile: the library's rule (gr_gemm_f32_groups), matrix-core cycles per SIMD of
+    the launch's rounds below 0.8 of the tile's (nk k tiles over four groups) and
+    at most two rounds per block that a wave of the tile owns (three where it
+    owns one and B is not K-major; four on a tile of two waves). 64 x 64 tiles with K = 1024: 256 x 512 (32 of
+    them) 25.1 -> 7.1 us, 512 x 1024 (128) 25.6 -> 17, 1024 x 1024 (256) 26 -> 33."""
     waves = (2 if bm >= 64 else 1) * (2 if bn >= 64 else 1)
     chain = (bm // 32) * (bn // 32) // waves            # 32 x 32 blocks per wave, nk k tiles each
-    tiles, blocks = batch * _cdiv(M, bm) * _cdiv(N, bn), batch * (M // 32) * (N // 32)
-    return 10 * _cdiv(blocks, cus) * (_cdiv(nk, 4) + 1) < 7 * _cdiv(tiles, cus) * (chain * nk + 1)
+    tiles = batch * _cdiv(M, bm) * _cdiv(N, bn)
+    rounds = _cdiv(batch * (M // 32) * (N // 32), cus)
+    return rounds <= (4 * chain if waves == 2 else 2 * chain + (chain == 1 and not kmajor)) and \
+        10 * rounds * _cdiv(nk, 4) < 8 * _cdiv(tiles, cus) * chain * nk
 
 
 def _gemm_waves(bm, bn):
@@ -667,7 +670,7 @@ def _match_gemm(loop: ParallelLoop, program: Program):
         # "kgroups": 1 = the program's tile, 4 = the blocks)
         kg = int((getattr(loop, "knobs", None) or {}).get("kgroups", 0))
         if kg not in GEMM_KGROUPS:
-            kg = 4 if _gemm_f32_groups(M, N, K // min(BK, 16), batch, BM, BN) else 1
+            kg = 4 if _gemm_f32_groups(M, N, K // min(BK, 16), batch, kmajor, BM, BN) else 1
         return {"a": aload.source, "b": bload.source, "c": loop.out, "M": M, "N": N, "K": K, "batch": batch,
                 "a_sb": M * K if a_batched else 0, "b_sb": K * N if b_batched else 0, "c_sb": M * N,
                 "kmajor": kmajor, "act": act, "alpha": alpha, "BM": BM, "BN": BN, "BK": BK,

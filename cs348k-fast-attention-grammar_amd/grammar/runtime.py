@@ -107,7 +107,7 @@ def lib() -> ctypes.CDLL:
         L.gr_gemm_workspace.restype = sz
         L.gr_gemm_ws.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, _ll2, _ll2, _ll2, i32, i32,
                                  ctypes.c_float, vp, sz, vp]
-        L.gr_gemm_f32_groups.argtypes = [i32, i32, i32, i32, i32, i32, i32]
+        L.gr_gemm_f32_groups.argtypes = [i32] * 8
         L.gr_mlp_fwd.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp]
         L.gr_mlp_fwd_workspace.argtypes = [i32, i32, i32, i32]
         L.gr_mlp_fwd_workspace.restype = sz

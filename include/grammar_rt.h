@@ -273,7 +273,7 @@ int gr_gemm_ws(const void* a, const void* b, void* c, int dtype, int batch, int 
  * tiles of 16, or 8 where 16 does not divide it) as 32 x 32 blocks with K over the
  * four waves of a workgroup rather than on block_m x block_n tiles, on `cus`
  * compute units: 1 or 0. Rendered fp32 stages follow the same rule. No counterpart in the reference. */
-int gr_gemm_f32_groups(int batch, int M, int N, int ktiles, int block_m, int block_n, int cus);
+int gr_gemm_f32_groups(int batch, int M, int N, int ktiles, int b_kmajor, int block_m, int block_n, int cus);
 
 /* MLP block Y = SiLU(X @ W1) @ W2 as two GEMMs, SiLU fused into the first.
  * The grammar's MLP program (run_mlp_search.py:42-127, with silu in place of
