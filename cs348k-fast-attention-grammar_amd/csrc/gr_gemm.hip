@@ -324,19 +324,22 @@ int mlp_fwd(const void* x, const void* w1, const void* w2, void* h, void* y, int
 // k tiles, below 0.8 of the tile's; and few rounds, since blocks read their
 // operands without sharing them: up to two per 32 x 32 block that a wave of the
 // tile owns (a third where it owns one and B is not K-major), four where the tile
-// has two waves, which leave half of a CU's SIMDs idle. Over 11,054 pairs of shape
-// and tile (M, N 64-4096, K 32-2048; tiles of 32, 64, 128 a side) the choice is
-// within 0.6 % of the faster body (geometric mean; 2.3 % with the first line
-// alone, which took M 768, N 4096, K 1024 from 79 us on 128 x 128 to 98 and
-// 4096 x 512, K 64 K-major on 32 x 32 from 7.0 to 11.8).
+// has two waves, which leave half of a CU's SIMDs idle; from 32 k tiles on also
+// 2.5 per block of the tile's rounds of four waves per CU, the last of them
+// part-filled (960 x 1152, K 704 on 64 x 64 tiles: five rounds 29.5 us, the tile's
+// two 31.9). Over 11,054 pairs of shape and tile (M, N 64-4096, K 32-2048; tiles
+// of 32, 64, 128 a side) the choice is within 0.4 % of the faster body (geometric
+// mean; 2.3 % with the first line alone, which took M 768, N 4096, K 1024 from 79
+// us on 128 x 128 to 98 and 4096 x 512, K 64 K-major on 32 x 32 from 7.0 to 11.8).
 extern "C" int gr_gemm_f32_groups(int batch, int M, int N, int ktiles, int b_kmajor, int block_m, int block_n, int cus) {
   if (batch <= 0 || M <= 0 || N <= 0 || ktiles <= 0 || block_m < 32 || block_n < 32 || cus <= 0) return 0;
   const int waves = (block_m >= 64 ? 2 : 1) * (block_n >= 64 ? 2 : 1);
   const long long tiles = (long long)batch * ((M + block_m - 1) / block_m) * ((N + block_n - 1) / block_n);
   const long long blocks = (long long)batch * (M / 32) * (N / 32);
   const long long chain = (long long)(block_m / 32) * (block_n / 32) / waves;       // 32 x 32 blocks per wave
-  const long long rounds = (blocks + cus - 1) / cus;
-  if (rounds > (waves == 2 ? 4 * chain : 2 * chain + (chain == 1 && !b_kmajor))) return 0;
+  const long long rounds = (blocks + cus - 1) / cus, full = (tiles * waves + 4LL * cus - 1) / (4LL * cus);
+  const long long few = waves == 2 ? 4 * chain : 2 * chain + (chain == 1 && !b_kmajor);
+  if (rounds > few && (ktiles < 32 || 2 * rounds > 5 * chain * full)) return 0;
   return 10 * rounds * ((ktiles + 3) / 4) < 8 * ((tiles + cus - 1) / cus) * chain * ktiles;
 }
 

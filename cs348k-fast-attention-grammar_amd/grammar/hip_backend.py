@@ -538,15 +538,17 @@ def _gemm_f32_groups(M, N, nk, batch, kmajor, bm, bn, cus=GEMM_CUS):
     waves of a workgroup (gr_gemm_f32_groups_body) instead of the program's
     tile: the library's rule (gr_gemm_f32_groups), matrix-core cycles per SIMD of
     the launch's rounds below 0.8 of the tile's (nk k tiles over four groups) and
-    at most two rounds per block that a wave of the tile owns (three where it
-    owns one and B is not K-major; four on a tile of two waves). 64 x 64 tiles with K = 1024: 256 x 512 (32 of
-    them) 25.1 -> 7.1 us, 512 x 1024 (128) 25.6 -> 17, 1024 x 1024 (256) 26 -> 33."""
+    few rounds, by the blocks that a wave of the tile owns. 64 x 64 tiles with K =
+    1024: 256 x 512 (32 of them) 25.1 -> 7.1 us, 512 x 1024 (128) 25.6 -> 17, 1024
+    x 1024 (256) 26 -> 33."""
     waves = (2 if bm >= 64 else 1) * (2 if bn >= 64 else 1)
     chain = (bm // 32) * (bn // 32) // waves            # 32 x 32 blocks per wave, nk k tiles each
     tiles = batch * _cdiv(M, bm) * _cdiv(N, bn)
-    rounds = _cdiv(batch * (M // 32) * (N // 32), cus)
-    return rounds <= (4 * chain if waves == 2 else 2 * chain + (chain == 1 and not kmajor)) and \
-        10 * rounds * _cdiv(nk, 4) < 8 * _cdiv(tiles, cus) * chain * nk
+    rounds, full = _cdiv(batch * (M // 32) * (N // 32), cus), _cdiv(tiles * waves, 4 * cus)
+    few = 4 * chain if waves == 2 else 2 * chain + (chain == 1 and not kmajor)
+    if rounds > few and (nk < 32 or 2 * rounds > 5 * chain * full):
+        return False
+    return 10 * rounds * _cdiv(nk, 4) < 8 * _cdiv(tiles, cus) * chain * nk
 
 
 def _gemm_waves(bm, bn):

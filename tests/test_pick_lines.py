@@ -39,6 +39,8 @@ def test_rendered_fp32_stages_follow_the_library_rule():
     (256, 512, 64, False, 64, 64, True), (512, 1024, 64, True, 64, 64, True), (1024, 1024, 64, False, 64, 64, False),
     (640, 1152, 32, False, 64, 64, True),          # three rounds of blocks: 46.4 us the whole program, 47.3 on the tile
     (640, 1152, 32, True, 64, 64, False),          # K-major
+    (960, 1152, 44, False, 32, 32, True), (960, 1152, 44, True, 64, 64, True),    # five rounds against two part-filled ones
+    (960, 1152, 16, False, 64, 64, False), (1024, 1024, 44, False, 32, 32, False), (1024, 1536, 44, False, 64, 64, False),
     (1024, 512, 4, True, 32, 32, True), (1024, 2048, 4, True, 32, 32, False),     # 8 rounds: 11.6 us, 7.1 on the tile
     (768, 4096, 64, False, 128, 128, False),       # 12 rounds: 98 us, 79 on the tile
     (2048, 1024, 16, False, 128, 128, True), (1536, 1408, 12, True, 128, 128, False),
