@@ -9,12 +9,14 @@
 // N = 512, d = 64: 67 MFLOP). At the fp32 matrix cores' rate one wave takes
 // about 2 us per 32 x 32 block of queries x keys, so the work is spread as
 // wide as the problem allows. A workgroup owns one 32-query block and NW
-// consecutive chunks of BN keys, one per wave; a wave runs the online softmax
-// over its chunk's 32-key blocks with its operands read straight from global
-// memory into registers (the next block's loads in flight during this
-// block's MFMAs). The NW partials (O, m, l) are merged through LDS, each wave
-// merging a D / NW slice. With PARTS = N / (NW BN) > 1 workgroups per query
-// block, each leaves its merged partial in a workspace and a second launch
+// consecutive runs of 32-key blocks, one per wave; a wave runs the online softmax
+// over its run with its operands read straight from global memory into registers
+// (the next block's K in flight during this block's MFMAs). The runs are BN / 32
+// blocks each in rendered stages (there PARTS = N / (NW BN)); behind gr_attn_fwd
+// the call's N / 32 blocks are shared out over the NW PARTS waves in runs that
+// differ by at most one. The NW partials (O, m, l) are merged through LDS, each
+// wave merging a D / NW slice. With PARTS > 1 workgroups per query block, each
+// leaves its merged partial in a workspace and a second launch
 // (gr_flash32_merge_body) combines them,
 //   O = sum_s 2^((m_s - M) c) O_s / sum_s 2^((m_s - M) c) l_s,  M = max_s m_s.
 // The workspace is module-scope device arrays the renderer sizes for the

@@ -190,10 +190,11 @@ int gr_attn_bwd(const void* q, const void* k, const void* v, const void* o, cons
  *  Q, O: [B, H, Nq, D]; K, V: [B, H, N, D]; strides {batch, head, seq} in
  *  elements (multiples of 8), unit stride along D. N a multiple of 32; D in
  *  {64, 128}; dtype GR_F16 or GR_BF16.
- *  With GR_F16 and more than 4 queries, scale * log2(e) must be <= 1 (as for
- *  gr_attn_fwd; GR_E_ARG otherwise).
  *  Up to 4 queries run on a streaming kernel (K and V read once straight
- *  into registers, scores on the VALU); more on the flash body's MFMA tiles.
+ *  into registers, scores on the VALU); more on the flash body's MFMA tiles,
+ *  up to 64 of them with four key groups inside the workgroup. With GR_F16,
+ *  more than 4 queries and scale * log2(e) > 1, Q is kept as given (as by
+ *  gr_attn_fwd) and a workgroup is one wave of 32 queries without groups.
  *  splits: workgroups per head (up to 4 queries) or per query tile that
  *  share out the keys (clamped to N/32, or to the number of 64- or 32-key
  *  tiles); with more than one, the partials go
